@@ -651,17 +651,25 @@ __global__ __launch_bounds__(256) void k_max_top(ChunkView cv, uint8_t* __restri
   }
 }
 
+// A wave probes T tiles (1 .. 64, chosen by launch_max so that the waves of the
+// grid share the tiles evenly), tile k * nwaves + wave in lane k: the kernel is
+// bound by the serial rebuilds of one wave, each a dependent round of loads
+// (about 1 us), and not by the probes, so neither a column whose tiles nearly
+// all hold the top byte (uniform values) nor a run of such tiles (a walk near
+// its maximum) may fall to few waves. With 64 consecutive tiles per wave a
+// 1,048,576-row uniform column took 106 us on 16 waves (6 us now) and a
+// 134,217,728-row walk 14.9 us (4.8 now).
 __global__ __launch_bounds__(256) void k_max_refine(ChunkView cv, const uint8_t* __restrict__ tile_max,
-                                                    const unsigned int* __restrict__ slots, uint32_t tag,
+                                                    const unsigned int* __restrict__ slots, uint32_t tag, uint32_t T,
                                                     unsigned long long* __restrict__ best_out) {
   const uint32_t lane = __lane_id();
   const uint64_t wave = wave_global();
   const uint64_t nwaves = waves_in_grid();
   const bool has_planes = cv.P > 0;
-  // 64 tiles per probe, one byte per lane; the first probe's bytes are loaded
+  // T tiles per probe, one byte per lane; the first probe's bytes are loaded
   // together with the slots
-  uint64_t base = wave * 64;
-  uint32_t tm = (has_planes && base + lane < cv.ntiles) ? tile_max[base + lane] : 0u;
+  uint64_t c = lane * nwaves + wave;
+  uint32_t tm = (has_planes && lane < T && c < cv.ntiles) ? tile_max[c] : 0u;
   uint32_t t = 0;
   if (has_planes) {
     const uint32_t m = wave_max_u32_dpp(slots[lane]);   // one slot per lane
@@ -669,16 +677,15 @@ __global__ __launch_bounds__(256) void k_max_refine(ChunkView cv, const uint8_t*
   }
   uint64_t best = 0;
   bool have = false;
-  for (; base < cv.ntiles; base += nwaves * 64) {
-    const uint64_t c = base + lane;
-    const bool hit = c < cv.ntiles && (!has_planes || tm == t);
-    const uint64_t nb = base + nwaves * 64;
-    tm = (has_planes && nb + lane < cv.ntiles) ? tile_max[nb + lane] : 0u;   // the next probe's bytes
+  for (uint64_t base = wave; base < cv.ntiles; base += nwaves * T, c += nwaves * T) {
+    const bool hit = lane < T && c < cv.ntiles && (!has_planes || tm == t);
+    const uint64_t nc = c + nwaves * T;
+    tm = (has_planes && lane < T && nc < cv.ntiles) ? tile_max[nc] : 0u;   // the next probe's bytes
     uint64_t hits = __ballot(hit);
     while (hits) {
       const uint32_t k = (uint32_t)__builtin_ctzll(hits);
       hits &= hits - 1;
-      const uint64_t ct = base + k;
+      const uint64_t ct = base + k * nwaves;
       // every plane and tail bit-plane of the tile in flight together
       uint4 wp[kMaxPlanes];
       uint32_t th[7];
@@ -711,7 +718,15 @@ __global__ __launch_bounds__(256) void k_max_refine(ChunkView cv, const uint8_t*
       have = true;
     }
   }
-  if (have && lane == 0) atomicMax(best_out, (unsigned long long)best);
+  // one update per workgroup, and only while it raises the result: device
+  // atomics on one address serialize (about 11 ns each)
+  __shared__ unsigned long long wbest[4];
+  if (lane == 0) wbest[wave_in_wg()] = have ? best + 1 : 0;
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    const unsigned long long b = max(max(wbest[0], wbest[1]), max(wbest[2], wbest[3]));
+    if (b && b - 1 > __hip_atomic_load(best_out, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) atomicMax(best_out, b - 1);
+  }
 }
 
 // One pass (a tuner choice; the two-pass form below is the default): every
@@ -1347,8 +1362,11 @@ hipError_t launch_max(const ChunkView& cv, unsigned long long* best, uint8_t* sc
       default: launch_max_top_u<8>(cv, scratch, slots, tag, best, s, ls); break;
     }
   }
-  const uint32_t wg2 = std::min(grid_for((cv.ntiles + 63) / 64, 4, 1024), resident_wgs(k_max_refine, 256));
-  launch_k(k_max_refine, dim3(wg2), dim3(256), 0, s, cv, (const uint8_t*)scratch, (const unsigned int*)slots, tag,
+  const uint32_t fit = resident_wgs(k_max_refine, 256);
+  uint32_t T = 1;   // tiles per wave: the fewest with which every wave is resident
+  while (T < 64 && (cv.ntiles + T - 1) / T > 4ull * fit) T *= 2;
+  const uint32_t wg2 = grid_for((cv.ntiles + T - 1) / T, 4, fit);
+  launch_k(k_max_refine, dim3(wg2), dim3(256), 0, s, cv, (const uint8_t*)scratch, (const unsigned int*)slots, tag, T,
            best);
   return hipGetLastError();
 }
