@@ -74,11 +74,14 @@ struct BResult {
 // Device-side counters of the current batch (written with the descriptors).
 // Items [0, nscan) are filters, sums and maxima; [nscan, nitems) materializations.
 // The host assigns every query its item range (item0, nitems) and the first
-// kernel of the batch writes the items themselves (tiles_per_item tiles each).
+// kernel of the batch writes the items themselves (tiles_per_item tiles each, a
+// materialization's mat_tiles).
 struct BHeader {
   uint32_t nq, nitems;
   uint32_t nscan;
   uint32_t tiles_per_item;
+  uint32_t mat_tiles;
+  uint32_t pad;
 };
 
 struct BatchBuffers {
@@ -106,6 +109,9 @@ struct BatchTuning {
   uint32_t tiles_per_item;
   uint32_t pad;
 };
+
+// Workgroups of the materialization kernels: four fit a CU's LDS.
+constexpr uint32_t kMatGrid = 1024;
 
 constexpr uint64_t kHostQueries = 256;   // byte offset of the queries in host_in
 

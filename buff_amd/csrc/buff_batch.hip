@@ -459,14 +459,16 @@ __global__ __launch_bounds__(256) void k_bq_publish(const BatchBuffers* __restri
 }
 
 // One workgroup per query: writes the query's work items (tile ranges of
-// tiles_per_item tiles over its chunk) at the range the host assigned it.
+// tiles_per_item or mat_tiles tiles over its chunk) at the range the host
+// assigned it.
 __global__ __launch_bounds__(256) void k_bq_items(const BatchBuffers* __restrict__ bbp) {
   const BatchBuffers bb = cload(bbp);
   const uint32_t nq = cmem(bb.hdr)->nq;
-  const uint64_t T = cmem(bb.hdr)->tiles_per_item;
+  const uint64_t Tscan = cmem(bb.hdr)->tiles_per_item, Tmat = cmem(bb.hdr)->mat_tiles;
   for (uint32_t qi = blockIdx.x; qi < nq; qi += gridDim.x) {
     const BQuery q = cload(bb.q, qi);
     if (!q.nitems) continue;
+    const uint64_t T = q.op == kBqMat ? Tmat : Tscan;
     const uint64_t ntiles = cmem(&bb.views[q.chunk].ntiles)[0];
     for (uint32_t j = threadIdx.x; j < q.nitems; j += blockDim.x) {
       const uint64_t c0 = (uint64_t)j * T;
@@ -873,10 +875,9 @@ hipError_t launch_batch_queries(const BatchBuffers* bb, const BatchTuning& tu, u
     hipLaunchKernelGGL(k_bq_max_refine, dim3(tu.grid), dim3(256), 0, s, bb);
     hipLaunchKernelGGL(k_bq_max_final, dim3(256), dim3(256), 0, s, bb);
   }
-  // four resident workgroups per CU fit the LDS staging of k_bq_mat
-  if (parts & kBqPartMat) hipLaunchKernelGGL(k_bq_mat, dim3(tu.grid < 1024 ? tu.grid : 1024), dim3(256), 0, s, bb);
-  if (parts & kBqPartMajorMat)
-    hipLaunchKernelGGL(k_bq_major_mat, dim3(tu.grid < 1024 ? tu.grid : 1024), dim3(256), 0, s, bb);
+  const uint32_t mat_grid = tu.grid < kMatGrid ? tu.grid : kMatGrid;
+  if (parts & kBqPartMat) hipLaunchKernelGGL(k_bq_mat, dim3(mat_grid), dim3(256), 0, s, bb);
+  if (parts & kBqPartMajorMat) hipLaunchKernelGGL(k_bq_major_mat, dim3(mat_grid), dim3(256), 0, s, bb);
   hipLaunchKernelGGL(k_bq_publish, dim3(16), dim3(256), 0, s, bb);
   return hipGetLastError();
 }

@@ -383,7 +383,7 @@ int exec_launch(QueryExec& ex, const std::vector<Chunk*>& chunks, const void* vi
   const uint64_t Tmax = std::min<uint32_t>(std::max<uint32_t>(tu.tiles_per_item, 1), kMaxTilesPerItem);
   ex.hq.assign(nq, BQuery{});
   std::vector<uint64_t> qtiles(nq, 0);
-  uint64_t total_tiles = 0;
+  uint64_t scan_tiles = 0, mat_tiles = 0;
   ex.res_host.assign(nq, buff_query_result{});
   ex.nq = nq;
   ex.host_ops.clear();
@@ -497,12 +497,17 @@ int exec_launch(QueryExec& ex, const std::vector<Chunk*>& chunks, const void* vi
         tiles = false;
     }
     qtiles[k] = tiles ? v.ntiles : 0;
-    total_tiles += qtiles[k];
+    (q.op == kBqMat ? mat_tiles : scan_tiles) += qtiles[k];
   }
   // Item length: the tuned one, shortened when the batch has too few tiles to
-  // give every wave of the grid (4 per workgroup) an item.
+  // give every wave of the kernel's grid (4 per workgroup) an item. Scans and
+  // materializations are counted apart: 64 materializations of 150k rows among
+  // 4096 queries made 150 items of the scans' 64 tiles, 154 us on 150 of the
+  // 4096 waves.
   const uint64_t waves = 4ull * std::max<uint32_t>(tu.grid, 1);
-  const uint64_t T = std::max<uint64_t>(1, std::min<uint64_t>(Tmax, (total_tiles + waves - 1) / waves));
+  const uint64_t mat_waves = std::min<uint64_t>(waves, 4ull * kMatGrid);
+  const uint64_t T = std::max<uint64_t>(1, std::min<uint64_t>(Tmax, (scan_tiles + waves - 1) / waves));
+  const uint64_t Tm = std::max<uint64_t>(1, std::min<uint64_t>(Tmax, (mat_tiles + mat_waves - 1) / mat_waves));
   // item ranges: scan items first, materializations after them (their item0 is
   // rebased below); k_bq_items writes the items on the device
   uint64_t n_scan = 0, n_mat = 0;
@@ -510,7 +515,8 @@ int exec_launch(QueryExec& ex, const std::vector<Chunk*>& chunks, const void* vi
     BQuery& q = ex.hq[k];
     uint64_t& next = q.op == kBqMat ? n_mat : n_scan;
     q.item0 = (uint32_t)next;
-    q.nitems = (uint32_t)((qtiles[k] + T - 1) / T);
+    const uint64_t t = q.op == kBqMat ? Tm : T;
+    q.nitems = (uint32_t)((qtiles[k] + t - 1) / t);
     next += q.nitems;
   }
   if (n_scan + n_mat > 0xFFFFFFFFull) return fail(BUFF_E_INVALID, "batch work items exceed 2^32");
@@ -552,7 +558,7 @@ int exec_launch(QueryExec& ex, const std::vector<Chunk*>& chunks, const void* vi
     ex.bb_valid = true;
   }
   if (nq == 0) return BUFF_OK;
-  ex.h = BHeader{nq, nitems, nscan, (uint32_t)T};
+  ex.h = BHeader{nq, nitems, nscan, (uint32_t)T, (uint32_t)Tm, 0};
   memcpy(ex.pin, &ex.h, sizeof(ex.h));
   memcpy(ex.pin + pin_queries_off(), ex.hq.data(), sizeof(BQuery) * nq);
   uint32_t parts = 0;
