@@ -919,6 +919,11 @@ int max_range_device(Ctx* ctx, const Chunk* ch, uint64_t s, uint64_t e, uint64_t
     if (argmax && nwords) HIP_TRY(launch_fill_bitmap(argmax, nwords, ch->n, 0, ctx->stream));
     return BUFF_OK;
   }
+  if (W >= kWmaxBlockMin && W <= kWmaxBlockMax) {
+    ProfScope ps(ctx, "k_wmax");
+    HIP_TRY(launch_wmax_block(v, s, e, W, k, std::ldexp(1.0, -(int)ch->dlen), vals, want, argmax, ctx->stream));
+    return BUFF_OK;
+  }
   BUFF_TRY(ctx->scratch(ctx->s_wmax, lay.bytes));
   uint8_t* scr = (uint8_t*)ctx->s_wmax.ptr;
   ProfScope ps(ctx, "k_wmax");

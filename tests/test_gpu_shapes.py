@@ -35,3 +35,29 @@ def test_max_ties(ctx, rows, data):
     value, off = ch.max()
     assert off == want - info.base and value == want / 2.0 ** info.dlen
     ch.free()
+
+
+def bits(words, n):
+    return np.unpackbits(np.asarray(words, dtype="<u4").view(np.uint8), bitorder="little")[:n].astype(bool)
+
+
+# one launch for windows of 16 .. 8192 rows (one tile a wave up to 2048 tiles, then four); the general path around it
+@pytest.mark.parametrize("decimals,rows", [(1, 40), (1, 5000), (3, 70_001), (4, 2048 * TILE), (4, 2048 * TILE + 3),
+                                           (6, 2100 * TILE - 1)])
+@pytest.mark.parametrize("window", [15, 16, 17, 1000, 1023, 1024, 1025, 8192, 8193])
+def test_windowed_max(ctx, decimals, rows, window):
+    x = datagen.random_walk(rows, decimals, 21)
+    ch = ctx.encode(x, 10 ** decimals)
+    dlen = ch.info().dlen
+    f = fixed(x, dlen)
+    for s, e in {(0, rows), (min(17, rows - 1), rows), (rows // 3, rows - rows // 5), (min(1500, rows - 1), rows - 1)}:
+        if e <= s:
+            continue
+        vals, words = ch.max_range(s, e, window, flags=buff_amd.BUFF_SEMANTIC)
+        at = np.arange(0, e - s, window)
+        want = np.maximum.reduceat(f[s:e], at)
+        assert np.array_equal(vals, want / 2.0 ** dlen), (s, e)
+        hit = np.zeros(rows, dtype=bool)
+        hit[s:e] = f[s:e] == np.repeat(want, window)[: e - s]
+        assert np.array_equal(bits(words, rows), hit), (s, e)
+    ch.free()
