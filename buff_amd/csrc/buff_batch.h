@@ -59,12 +59,17 @@ struct BQuery {
   uint32_t fill;         // filters: 0 = run, 1 = no rows, 2 = all rows (decided on the host)
   uint32_t item0, nitems;
   uint32_t sparse;       // buff-major chunk with sparse columns: S (bits 0-7), BUFF_SEMANTIC (bit 8); else 0
-  FilterTarget tg;       // filters (on a buff-major chunk: the target byte of every byte column, sparse first)
-  MatParams mp;          // materialize (buff-major: mode kMatSemantic keeps the top F - drop bits)
-  uint64_t out;          // filters: device address of the ceil(n/64) bitmap words;
+  union {
+    FilterTarget tg;     // filters (on a buff-major chunk: the target byte of every byte column, sparse first)
+    MatParams mp;        // materialize (buff-major: mode kMatSemantic keeps the top F - drop bits)
+  };
+  union {
+    uint64_t out;        // filters: device address of the ceil(n/64) bitmap words;
                          // materialize: device address of the n doubles
-  uint64_t top;          // max: byte offset of its per-tile top bytes in the max arena
+    uint64_t top;        // max: byte offset of its per-tile top bytes in the max arena
+  };
 };
+static_assert(sizeof(BQuery) == 72, "BQuery: read over the bus once per query and batch");
 
 // Per-query results the host reads back.
 struct BResult {
@@ -72,21 +77,21 @@ struct BResult {
 };
 
 // Device-side counters of the current batch (written with the descriptors).
-// Items [0, nscan) are filters, sums and maxima; [nscan, nitems) materializations.
-// The host assigns every query its item range (item0, nitems) and the first
-// kernel of the batch writes the items themselves (tiles_per_item tiles each, a
-// materialization's mat_tiles).
+// Items [0, max0) are sums, then filters; [max0, nscan) maxima; [nscan, nitems)
+// materializations. The host assigns every query its item range (item0, nitems)
+// and the first kernel of the batch writes the items themselves (tiles_per_item
+// tiles each, a materialization's mat_tiles).
 struct BHeader {
   uint32_t nq, nitems;
   uint32_t nscan;
   uint32_t tiles_per_item;
   uint32_t mat_tiles;
-  uint32_t pad;
+  uint32_t max0;
 };
 
 struct BatchBuffers {
   const uint8_t* host_in;            // pinned host: BHeader at 0, nq BQuery at kHostQueries
-  BResult* host_res;                 // pinned host: nq results, written by the last kernel
+  BResult* host_res;                 // pinned host: nq results, written as they are folded
   const BHeader* hdr;
   const ChunkView* views;
   const MajorView* majors;           // per chunk, read only by queries whose chunk has sparse columns
@@ -94,7 +99,7 @@ struct BatchBuffers {
   BItem* items;                      // written by the batch's first kernel
   uint8_t* tile_top;                 // max: per-tile top byte
   unsigned long long* item_acc;      // per item: kMaxPlanes + 1 u64
-  BResult* res;
+  BResult* res;                      // maxima: v[0] the max offset, v[1] the top byte
 };
 
 // `grid` is the persistent grid size and `tiles_per_item` the work item length

@@ -128,18 +128,18 @@ hipError_t launch_batch_encode(const BEncChunk* chunks, const BItem* items, uint
 // ----------------------------------------------------------------------------
 // Batch queries. One wave works on one item at a time (items of different
 // queries interleave freely; the item loops hold no workgroup barrier):
-//   k_bq_fetch  copies the header and query descriptors from pinned host memory;
-//   k_bq_items  writes the work items from the per-query item ranges;
+//   k_bq_fetch  copies the header and query descriptors from pinned host memory
+//               and writes the work items from the per-query item ranges;
 //   k_bq_scan   items [0, nscan): filters write tile bitmaps and count them,
 //               sums add the sub-column bytes and tail bits, maxima record every
 //               tile's top byte;
-//   k_bq_reduce one wave per query folds its items' partials;
-//   k_bq_max_refine / k_bq_max_final: the tiles holding a max query's top byte
-//               give its max offset;
+//   k_bq_reduce one wave per query folds its items' partials and writes the
+//               result to pinned host memory;
+//   k_bq_max_refine the tiles holding a max query's top byte give its max offset;
 //   k_bq_mat    items [nscan, nitems): materializations, staged through LDS for
 //               coalesced f64 stores (kept apart so the scan kernel holds no LDS
 //               and runs at full occupancy);
-//   k_bq_publish copies the results to pinned host memory.
+//   k_bq_max_publish writes the maxima to pinned host memory.
 // Per-tile loads are issued together: a filter reads the top byte plane, then
 // every remaining plane and tail bit-plane of the tied rows at once; sums and
 // materializations read all their planes before combining them.
@@ -305,30 +305,6 @@ __device__ __forceinline__ void sum_item(const ChunkView& cv, const BItem& it, u
   for (uint64_t c = it.c0; c < it.c1; ++c) sum_planes<0, NP>(cv, c, lane, acc);
 }
 
-// Max stored offset among the lane's 16 rows (rows >= n are zero): the max
-// byte plane by plane among the rows tying so far, then bit by bit on the tail.
-__device__ __forceinline__ uint64_t lane_offset_max(const ChunkView& cv, uint64_t c, uint32_t lane) {
-  uint32_t cand = 0xFFFFu;
-  uint64_t m = 0;
-#pragma unroll 1
-  for (uint32_t p = 0; p < cv.P; ++p) {
-    const uint4 w = load_plane(cv, p, c, lane);
-    const uint32_t mb = masked_max_plus1(w, cand) - 1u;   // cand is never empty
-    cand &= mask_eq(w, make_digit(mb));
-    m = (m << 8) | mb;
-  }
-#pragma unroll 1
-  for (uint32_t j0 = cv.r; j0 > 0; --j0) {
-    const uint32_t h = load_tail(cv, j0 - 1, c, lane) & cand;
-    m <<= 1;
-    if (h) {
-      m |= 1u;
-      cand = h;
-    }
-  }
-  return m;
-}
-
 // F < 8: the lane's max value from the tail bit-planes alone.
 __device__ __forceinline__ uint32_t lane_tail_max(const ChunkView& cv, uint64_t c, uint32_t lane) {
   uint32_t cand = 0xFFFFu, m = 0;
@@ -342,10 +318,6 @@ __device__ __forceinline__ uint32_t lane_tail_max(const ChunkView& cv, uint64_t 
     }
   }
   return m;
-}
-
-__device__ __forceinline__ uint64_t tile_offset_max(const ChunkView& cv, uint64_t c, uint32_t lane) {
-  return wave_max_u64(lane_offset_max(cv, c, lane));
 }
 
 __device__ __forceinline__ uint32_t lane_max_byte(const uint4& w) {
@@ -431,151 +403,136 @@ __global__ __launch_bounds__(256) void k_bq_scan(const BatchBuffers* __restrict_
 
 // Copies the batch's header and query descriptors from pinned host memory to
 // device memory (the host only writes them and launches the graph: no runtime
-// copy, which could queue behind another slot's transfers).
+// copy, which could queue behind another slot's transfers), and writes each
+// query's work items (tile ranges of tiles_per_item or mat_tiles tiles over its
+// chunk) at the range the host assigned it. One wave per query, a descriptor
+// per load: all of them are on the bus together, so the kernel is bound by its
+// rate (4096 descriptors of 72 bytes) and two round trips.
 __global__ __launch_bounds__(256) void k_bq_fetch(const BatchBuffers* __restrict__ bbp) {
+  constexpr uint32_t kHeaderWords = sizeof(BHeader) / 4, kQueryWords = sizeof(BQuery) / 4;
+  static_assert(kHeaderWords + kQueryWords <= 64, "one load per wave");
   const BatchBuffers bb = cload(bbp);
+  const WaveSlot ws = wave_slot();
+  const uint32_t lane = ws.lane;
   const BUFF_GLOBAL uint32_t* hin = gmem(reinterpret_cast<const uint32_t*>(bb.host_in));
-  BUFF_GLOBAL uint32_t* hdr = gmem_w(reinterpret_cast<uint32_t*>(const_cast<BHeader*>(bb.hdr)));
-  const uint32_t nq = hin[0];
-  const uint64_t tid = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x, nthreads = (uint64_t)gridDim.x * blockDim.x;
-  if (tid < sizeof(BHeader) / 4) hdr[tid] = hin[tid];
-  const uint64_t nwords = (uint64_t)nq * (sizeof(BQuery) / 4);
-  const BUFF_GLOBAL uint32_t* src = hin + kHostQueries / 4;
-  BUFF_GLOBAL uint32_t* dst = gmem_w(reinterpret_cast<uint32_t*>(const_cast<BQuery*>(bb.q)));
-  for (uint64_t i = tid; i < nwords; i += nthreads) dst[i] = src[i];
-}
-
-// Writes the batch's results to pinned host memory, visible to the host once
-// the batch's completion event has fired.
-__global__ __launch_bounds__(256) void k_bq_publish(const BatchBuffers* __restrict__ bbp) {
-  const BatchBuffers bb = cload(bbp);
-  const uint32_t nq = cmem(bb.hdr)->nq;
-  const uint64_t nwords = (uint64_t)nq * (sizeof(BResult) / 8);
-  const BUFF_GLOBAL uint64_t* src = gmem(reinterpret_cast<const uint64_t*>(bb.res));
-  BUFF_GLOBAL uint64_t* dst = gmem_w(reinterpret_cast<uint64_t*>(bb.host_res));
-  const uint64_t tid = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x, nthreads = (uint64_t)gridDim.x * blockDim.x;
-  for (uint64_t i = tid; i < nwords; i += nthreads) dst[i] = src[i];
-  __threadfence_system();
-}
-
-// One workgroup per query: writes the query's work items (tile ranges of
-// tiles_per_item or mat_tiles tiles over its chunk) at the range the host
-// assigned it.
-__global__ __launch_bounds__(256) void k_bq_items(const BatchBuffers* __restrict__ bbp) {
-  const BatchBuffers bb = cload(bbp);
-  const uint32_t nq = cmem(bb.hdr)->nq;
-  const uint64_t Tscan = cmem(bb.hdr)->tiles_per_item, Tmat = cmem(bb.hdr)->mat_tiles;
-  for (uint32_t qi = blockIdx.x; qi < nq; qi += gridDim.x) {
-    const BQuery q = cload(bb.q, qi);
-    if (!q.nitems) continue;
-    const uint64_t T = q.op == kBqMat ? Tmat : Tscan;
-    const uint64_t ntiles = cmem(&bb.views[q.chunk].ntiles)[0];
-    for (uint32_t j = threadIdx.x; j < q.nitems; j += blockDim.x) {
+  const uint32_t hw = lane < kHeaderWords ? hin[lane] : 0u;
+  if (ws.first == 0 && lane < kHeaderWords) gmem_w(reinterpret_cast<uint32_t*>(const_cast<BHeader*>(bb.hdr)))[lane] = hw;
+  const uint32_t nq = __builtin_amdgcn_readlane(hw, offsetof(BHeader, nq) / 4);
+  const uint32_t Tscan = __builtin_amdgcn_readlane(hw, offsetof(BHeader, tiles_per_item) / 4);
+  const uint32_t Tmat = __builtin_amdgcn_readlane(hw, offsetof(BHeader, mat_tiles) / 4);
+  for (uint32_t qi = ws.first; qi < nq; qi += ws.stride) {
+    const BUFF_GLOBAL uint32_t* src = hin + kHostQueries / 4 + (uint64_t)qi * kQueryWords;
+    const uint32_t w = lane < kQueryWords ? src[lane] : 0u;
+    if (lane < kQueryWords) gmem_w(reinterpret_cast<uint32_t*>(const_cast<BQuery*>(bb.q + qi)))[lane] = w;
+    const uint32_t op = __builtin_amdgcn_readlane(w, offsetof(BQuery, op) / 4);
+    const uint32_t chunk = __builtin_amdgcn_readlane(w, offsetof(BQuery, chunk) / 4);
+    const uint32_t item0 = __builtin_amdgcn_readlane(w, offsetof(BQuery, item0) / 4);
+    const uint32_t nitems = __builtin_amdgcn_readlane(w, offsetof(BQuery, nitems) / 4);
+    if (!nitems) continue;
+    const uint64_t T = op == kBqMat ? Tmat : Tscan;
+    const uint64_t ntiles = cmem(&bb.views[chunk].ntiles)[0];
+    for (uint32_t j = lane; j < nitems; j += 64) {
       const uint64_t c0 = (uint64_t)j * T;
-      BUFF_GLOBAL uint64_t* w = gmem_w(reinterpret_cast<uint64_t*>(bb.items + q.item0 + j));
-      w[0] = (uint64_t)qi | ((uint64_t)q.chunk << 32);   // owner, chunk
-      w[1] = c0;
-      w[2] = c0 + T < ntiles ? c0 + T : ntiles;
+      BUFF_GLOBAL uint64_t* it = gmem_w(reinterpret_cast<uint64_t*>(bb.items + item0 + j));
+      it[0] = (uint64_t)qi | ((uint64_t)chunk << 32);   // owner, chunk
+      it[1] = c0;
+      it[2] = c0 + T < ntiles ? c0 + T : ntiles;
     }
   }
 }
 
-// One workgroup per query folds its items' partials (filters: count, sums:
-// sub-column sums, maxima: the top byte into v[1]); each thread keeps four
-// partial rows in flight. Materializations have nothing to fold.
+// One wave per query folds its items' partials (filters: count, sums:
+// sub-column sums, maxima: the top byte), four partial rows in flight per lane,
+// and writes the result words to pinned host memory, visible to the host once
+// the batch's completion event has fired; a max query's top byte goes to device
+// memory for the refinement. Materializations have nothing to fold. (A
+// workgroup per query with its barriers and a separate copy of every result
+// took 29 + 11 us for 4096 queries.)
 __global__ __launch_bounds__(256) void k_bq_reduce(const BatchBuffers* __restrict__ bbp) {
-  __shared__ unsigned long long s_part[4][kMaxPlanes + 1];
   const BatchBuffers bb = cload(bbp);
-  const uint32_t lane = __lane_id(), wave = wave_in_wg();
+  const WaveSlot ws = wave_slot();
+  const uint32_t lane = ws.lane;
   const uint32_t nq = cmem(bb.hdr)->nq;
-  for (uint32_t qi = blockIdx.x; qi < nq; qi += gridDim.x) {
-    const BQuery q = cload(bb.q, qi);
-    const bool is_max = q.op == kBqMax;
-    const uint32_t nk = q.op == kBqSum ? kMaxPlanes + 1 : (q.op == kBqMat ? 0u : 1u);
+  for (uint32_t qi = ws.first; qi < nq; qi += ws.stride) {
+    const BUFF_CONST BQuery* q = cmem(bb.q + qi);
+    const uint32_t op = q->op, item0 = q->item0, nitems = q->nitems;
+    if (op == kBqMat) continue;
+    const bool is_max = op == kBqMax;
+    const uint32_t nk = op == kBqSum ? kMaxPlanes + 1 : 1u;
+    const BUFF_GLOBAL unsigned long long* acc = gmem(bb.item_acc) + (uint64_t)item0 * (kMaxPlanes + 1);
     unsigned long long v[kMaxPlanes + 1];
 #pragma unroll
     for (uint32_t k = 0; k <= kMaxPlanes; ++k) v[k] = 0;
-    const unsigned long long* acc = bb.item_acc + (uint64_t)q.item0 * (kMaxPlanes + 1);
-    for (uint32_t i0 = threadIdx.x; i0 < q.nitems; i0 += 4 * blockDim.x) {
+    for (uint32_t i0 = lane; i0 < nitems; i0 += 4 * 64) {
 #pragma unroll
       for (uint32_t k = 0; k <= kMaxPlanes; ++k) {
         if (k >= nk) continue;
         unsigned long long a[4];
 #pragma unroll
         for (uint32_t u = 0; u < 4; ++u) {
-          const uint32_t i = i0 + u * blockDim.x;
-          a[u] = i < q.nitems ? gmem(acc)[(uint64_t)i * (kMaxPlanes + 1) + k] : 0ull;
+          const uint32_t i = i0 + u * 64;
+          a[u] = i < nitems ? acc[(uint64_t)i * (kMaxPlanes + 1) + k] : 0ull;
         }
 #pragma unroll
         for (uint32_t u = 0; u < 4; ++u) v[k] = is_max ? max(v[k], a[u]) : v[k] + a[u];
       }
     }
+    unsigned long long mine = 0;   // lane k: result word k
 #pragma unroll
     for (uint32_t k = 0; k <= kMaxPlanes; ++k) {
       if (k >= nk) continue;
-      v[k] = is_max ? wave_max_u64(v[k]) : wave_sum_u64(v[k]);
-      if (lane == 0) s_part[wave][k] = v[k];
+      const unsigned long long t = is_max ? wave_max_u64(v[k]) : wave_sum_u64(v[k]);
+      if (lane == k) mine = t;
     }
-    __syncthreads();
-    if (threadIdx.x == 0) {
-      BResult r;
-#pragma unroll
-      for (uint32_t k = 0; k <= kMaxPlanes; ++k) {
-        unsigned long long t = 0;
-        if (k < nk) {
-          t = s_part[0][k];
-          for (uint32_t w = 1; w < (blockDim.x >> 6); ++w) t = is_max ? max(t, s_part[w][k]) : t + s_part[w][k];
-        }
-        r.v[k] = t;
+    if (is_max) {
+      // v[1] = the top byte; v[0] is raised by the refinement (a query without
+      // items has none: its result is the 0 written here)
+      if (lane == 0) {
+        bb.res[qi].v[0] = 0;
+        bb.res[qi].v[1] = mine;
+        gmem_w(bb.host_res[qi].v)[0] = 0;
       }
-      if (is_max) {
-        r.v[1] = r.v[0];   // top byte; v[0] is filled by the refine fold
-        r.v[0] = 0;
-      }
-      bb.res[qi] = r;
+    } else if (lane < nk) {
+      gmem_w(bb.host_res[qi].v)[lane] = mine;
     }
-    __syncthreads();
   }
 }
 
 // Maxima: tiles whose top byte equals the query's top byte give the max offset.
+// A wave probes 64 tiles of its item at once and rebuilds the ones that hold
+// the top byte, all planes of a tile in flight together.
 __global__ __launch_bounds__(256) void k_bq_max_refine(const BatchBuffers* __restrict__ bbp) {
   const BatchBuffers bb = cload(bbp);
   const WaveSlot ws = wave_slot();
   const uint32_t lane = ws.lane;
   const uint32_t nscan = cmem(bb.hdr)->nscan;
   #pragma unroll 1
-  for (uint32_t i = ws.first; i < nscan; i += ws.stride) {
+  for (uint32_t i = cmem(bb.hdr)->max0 + ws.first; i < nscan; i += ws.stride) {
     const BItem it = cload(bb.items, i);
-    const BQuery q = cload(bb.q, it.owner);
-    if (q.op != kBqMax) continue;
+    const uint64_t qtop = cmem(bb.q + it.owner)->top;
     const ChunkView cv = cload(bb.views, it.chunk);
     const uint32_t top = (uint32_t)cmem(bb.res[it.owner].v)[1];   // written by k_bq_reduce
-    unsigned long long best = 0;    // max offset + 1
+    uint64_t best = 0;
     #pragma unroll 1
-    for (uint64_t c = it.c0; c < it.c1; ++c) {
-      if (cmem(bb.tile_top)[q.top + c] != top) continue;   // written by k_bq_scan
-      const uint64_t m = tile_offset_max(cv, c, lane);
-      best = max(best, (unsigned long long)m + 1);
+    for (uint64_t c0 = it.c0; c0 < it.c1; c0 += 64) {
+      const uint64_t c = c0 + lane;
+      uint64_t hits = __ballot(c < it.c1 && gmem(bb.tile_top)[qtop + c] == top);   // written by k_bq_scan
+      while (hits) {
+        const uint64_t m = lane_max_offset(cv, c0 + (uint32_t)__builtin_ctzll(hits), lane);
+        hits &= hits - 1;
+        best = m > best ? m : best;
+      }
     }
-    if (lane == 0) bb.item_acc[(uint64_t)i * (kMaxPlanes + 1) + 1] = best;
+    best = wave_max_u64(best);
+    if (lane == 0 && best) atomicMax(&bb.res[it.owner].v[0], (unsigned long long)best);
   }
 }
 
-__global__ __launch_bounds__(256) void k_bq_max_final(const BatchBuffers* __restrict__ bbp) {
+__global__ __launch_bounds__(256) void k_bq_max_publish(const BatchBuffers* __restrict__ bbp) {
   const BatchBuffers bb = cload(bbp);
-  const WaveSlot ws = wave_slot();
-  const uint32_t lane = ws.lane;
   const uint32_t nq = cmem(bb.hdr)->nq;
-  for (uint32_t qi = ws.first; qi < nq; qi += ws.stride) {
-    const BQuery q = cload(bb.q, qi);
-    if (q.op != kBqMax) continue;
-    unsigned long long m = 0;
-    for (uint32_t i = lane; i < q.nitems; i += 64)
-      m = max(m, bb.item_acc[(uint64_t)(q.item0 + i) * (kMaxPlanes + 1) + 1]);
-    m = wave_max_u64(m);
-    if (lane == 0) bb.res[qi].v[0] = m ? m - 1 : 0;
-  }
+  for (uint32_t qi = blockIdx.x * blockDim.x + threadIdx.x; qi < nq; qi += gridDim.x * blockDim.x)
+    if (gmem(&bb.q[qi].op)[0] == kBqMax) gmem_w(bb.host_res[qi].v)[0] = gmem(bb.res[qi].v)[0];
 }
 
 // Materialize one tile from the top NP planes and mp.tail_bits tail bits below
@@ -864,21 +821,19 @@ __global__ __launch_bounds__(256) void k_bq_major_mat(const BatchBuffers* __rest
 }
 
 hipError_t launch_batch_queries(const BatchBuffers* bb, const BatchTuning& tu, uint32_t parts, hipStream_t s) {
-  hipLaunchKernelGGL(k_bq_fetch, dim3(64), dim3(256), 0, s, bb);
-  hipLaunchKernelGGL(k_bq_items, dim3(1024), dim3(256), 0, s, bb);
+  hipLaunchKernelGGL(k_bq_fetch, dim3(1024), dim3(256), 0, s, bb);
   if (parts & kBqPartScan) {
     hipLaunchKernelGGL(k_bq_scan, dim3(tu.grid), dim3(256), 0, s, bb, tu);
     if (parts & kBqPartMajor) hipLaunchKernelGGL(k_bq_major, dim3(tu.grid), dim3(256), 0, s, bb);
     hipLaunchKernelGGL(k_bq_reduce, dim3(1024), dim3(256), 0, s, bb);
   }
   if (parts & kBqPartMax) {
-    hipLaunchKernelGGL(k_bq_max_refine, dim3(tu.grid), dim3(256), 0, s, bb);
-    hipLaunchKernelGGL(k_bq_max_final, dim3(256), dim3(256), 0, s, bb);
+    hipLaunchKernelGGL(k_bq_max_refine, dim3(tu.grid < 2048 ? tu.grid : 2048), dim3(256), 0, s, bb);
+    hipLaunchKernelGGL(k_bq_max_publish, dim3(16), dim3(256), 0, s, bb);
   }
   const uint32_t mat_grid = tu.grid < kMatGrid ? tu.grid : kMatGrid;
   if (parts & kBqPartMat) hipLaunchKernelGGL(k_bq_mat, dim3(mat_grid), dim3(256), 0, s, bb);
   if (parts & kBqPartMajorMat) hipLaunchKernelGGL(k_bq_major_mat, dim3(mat_grid), dim3(256), 0, s, bb);
-  hipLaunchKernelGGL(k_bq_publish, dim3(16), dim3(256), 0, s, bb);
   return hipGetLastError();
 }
 

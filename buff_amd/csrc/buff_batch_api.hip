@@ -508,22 +508,30 @@ int exec_launch(QueryExec& ex, const std::vector<Chunk*>& chunks, const void* vi
   const uint64_t mat_waves = std::min<uint64_t>(waves, 4ull * kMatGrid);
   const uint64_t T = std::max<uint64_t>(1, std::min<uint64_t>(Tmax, (scan_tiles + waves - 1) / waves));
   const uint64_t Tm = std::max<uint64_t>(1, std::min<uint64_t>(Tmax, (mat_tiles + mat_waves - 1) / mat_waves));
-  // item ranges: scan items first, materializations after them (their item0 is
-  // rebased below); k_bq_items writes the items on the device
-  uint64_t n_scan = 0, n_mat = 0;
+  // item ranges, by operation: sums (the longest items) first, filters, maxima
+  // (whose refinement then reads only their own range), materializations;
+  // k_bq_fetch writes the items on the device
+  uint64_t next[4] = {0, 0, 0, 0};   // items per group, then each group's running position
+  auto group = [](const BQuery& q) { return q.op == kBqSum ? 0 : q.op == kBqMax ? 2 : q.op == kBqMat ? 3 : 1; };
   for (uint32_t k = 0; k < nq; ++k) {
     BQuery& q = ex.hq[k];
-    uint64_t& next = q.op == kBqMat ? n_mat : n_scan;
-    q.item0 = (uint32_t)next;
     const uint64_t t = q.op == kBqMat ? Tm : T;
     q.nitems = (uint32_t)((qtiles[k] + t - 1) / t);
-    next += q.nitems;
+    next[group(q)] += q.nitems;
   }
-  if (n_scan + n_mat > 0xFFFFFFFFull) return fail(BUFF_E_INVALID, "batch work items exceed 2^32");
-  const uint32_t nscan = (uint32_t)n_scan;
-  for (BQuery& q : ex.hq)
-    if (q.op == kBqMat) q.item0 += nscan;
-  const uint32_t nitems = (uint32_t)(n_scan + n_mat);
+  uint64_t total_items = 0;
+  for (uint64_t& n : next) {
+    const uint64_t count = n;
+    n = total_items;
+    total_items += count;
+  }
+  if (total_items > 0xFFFFFFFFull) return fail(BUFF_E_INVALID, "batch work items exceed 2^32");
+  const uint32_t nitems = (uint32_t)total_items, max0 = (uint32_t)next[2], nscan = (uint32_t)next[3];
+  for (BQuery& q : ex.hq) {
+    uint64_t& at = next[group(q)];
+    q.item0 = (uint32_t)at;
+    at += q.nitems;
+  }
   BUFF_TRY(ensure(ctx, ex.hdr, sizeof(BHeader)));
   BUFF_TRY(ensure(ctx, ex.q, sizeof(BQuery) * std::max<uint32_t>(nq, 1)));
   BUFF_TRY(ensure(ctx, ex.items, sizeof(BItem) * std::max<uint32_t>(nitems, 1)));
@@ -536,7 +544,7 @@ int exec_launch(QueryExec& ex, const std::vector<Chunk*>& chunks, const void* vi
     if (ex.res_host[k].status != BUFF_OK) continue;
     const uint64_t addr = (outs && outs[k]) ? outs[k] : (uint64_t)ex.arena.p + (arena_at[k] == ~0ull ? 0 : arena_at[k]);
     const bool has_out = qs[k].op == BUFF_Q_GT || qs[k].op == BUFF_Q_EQ || qs[k].op == BUFF_Q_MAT;
-    ex.hq[k].out = addr;
+    if (has_out) ex.hq[k].out = addr;
     ex.res_host[k].out_offset = has_out ? addr : 0;
   }
   BUFF_TRY(pin_reserve(ex, nq));
@@ -558,7 +566,7 @@ int exec_launch(QueryExec& ex, const std::vector<Chunk*>& chunks, const void* vi
     ex.bb_valid = true;
   }
   if (nq == 0) return BUFF_OK;
-  ex.h = BHeader{nq, nitems, nscan, (uint32_t)T, (uint32_t)Tm, 0};
+  ex.h = BHeader{nq, nitems, nscan, (uint32_t)T, (uint32_t)Tm, max0};
   memcpy(ex.pin, &ex.h, sizeof(ex.h));
   memcpy(ex.pin + pin_queries_off(), ex.hq.data(), sizeof(BQuery) * nq);
   uint32_t parts = 0;

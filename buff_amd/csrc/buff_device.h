@@ -242,6 +242,23 @@ struct RowBytes {
   uint32_t T[4];   // tail byte of row 4k + i in byte k of T[i]
 };
 
+// The r tail bit-planes h of the lane's 16 rows spread into the plane layout:
+// the tail byte of row 4k + i in byte k of T[i], bit j of the tail at bit 8 - r + j.
+template <uint32_t N>
+__device__ __forceinline__ void tail_bytes(const uint32_t (&h)[N], uint32_t r, uint32_t (&T)[4]) {
+  T[0] = T[1] = T[2] = T[3] = 0u;
+#pragma unroll
+  for (uint32_t j = 0; j < N; ++j) {
+    if (j >= r) break;
+    const uint32_t x = h[j];
+    // nibble k of the 16 row bits -> byte k
+    const uint32_t y = (x & 0xFu) | ((x << 4) & 0xF00u) | ((x << 8) & 0xF0000u) | ((x << 12) & 0xF000000u);
+    const uint32_t sh = 8u - r + j;
+#pragma unroll
+    for (uint32_t i = 0; i < 4; ++i) T[i] |= ((y >> i) & 0x01010101u) << sh;
+  }
+}
+
 template <int NP>
 __device__ __forceinline__ void load_row_bytes(const ChunkView& cv, uint64_t c, uint32_t src, RowBytes<NP>& rb) {
 #pragma unroll
@@ -250,17 +267,7 @@ __device__ __forceinline__ void load_row_bytes(const ChunkView& cv, uint64_t c, 
   uint32_t h[7];
 #pragma unroll
   for (uint32_t j = 0; j < 7; ++j) h[j] = j < r ? load_tail(cv, j, c, src) : 0u;
-  rb.T[0] = rb.T[1] = rb.T[2] = rb.T[3] = 0u;
-#pragma unroll
-  for (uint32_t j = 0; j < 7; ++j) {
-    if (j >= r) break;
-    const uint32_t x = h[j];
-    // nibble k of the 16 row bits -> byte k
-    const uint32_t y = (x & 0xFu) | ((x << 4) & 0xF00u) | ((x << 8) & 0xF0000u) | ((x << 12) & 0xF000000u);
-    const uint32_t sh = 8u - r + j;
-#pragma unroll
-    for (uint32_t i = 0; i < 4; ++i) rb.T[i] |= ((y >> i) & 0x01010101u) << sh;
-  }
+  tail_bytes<7>(h, r, rb.T);
 }
 
 // X of row b (see above): byte 0 the tail byte, bytes 1.. the planes from the last.
@@ -392,6 +399,38 @@ __device__ __forceinline__ uint32_t masked_max_plus1(const uint4& w, uint32_t ma
 #pragma unroll
   for (uint32_t b = 0; b < 16; ++b) v = ((mask >> b) & 1u) ? max(v, byte_at(w, b) + 1u) : v;
   return v;
+}
+
+// Max stored offset among the lane's 16 rows of tile c (rows >= n are zero):
+// every plane and tail bit-plane of the tile in flight together.
+__device__ __forceinline__ uint64_t lane_max_offset(const ChunkView& cv, uint64_t c, uint32_t lane) {
+  uint4 wp[kMaxPlanes];
+  uint32_t th[7];
+#pragma unroll
+  for (uint32_t p = 0; p < kMaxPlanes; ++p) wp[p] = p < cv.P ? load_plane(cv, p, c, lane) : make_uint4(0, 0, 0, 0);
+#pragma unroll
+  for (uint32_t j = 0; j < 7; ++j) th[j] = j < cv.r ? load_tail(cv, j, c, lane) : 0u;
+  uint64_t off[16];
+#pragma unroll
+  for (uint32_t b = 0; b < 16; ++b) off[b] = 0;
+#pragma unroll
+  for (uint32_t p = 0; p < kMaxPlanes; ++p) {
+    if (p < cv.P) {
+#pragma unroll
+      for (uint32_t b = 0; b < 16; ++b) off[b] = (off[b] << 8) | byte_at(wp[p], b);
+    }
+  }
+#pragma unroll
+  for (int j = 6; j >= 0; --j) {
+    if ((uint32_t)j < cv.r) {
+#pragma unroll
+      for (uint32_t b = 0; b < 16; ++b) off[b] = (off[b] << 1) | ((th[j] >> b) & 1u);
+    }
+  }
+  uint64_t m = 0;
+#pragma unroll
+  for (uint32_t b = 0; b < 16; ++b) m = off[b] > m ? off[b] : m;
+  return m;
 }
 
 }  // namespace buffgpu

@@ -686,34 +686,7 @@ __global__ __launch_bounds__(256) void k_max_refine(ChunkView cv, const uint8_t*
       const uint32_t k = (uint32_t)__builtin_ctzll(hits);
       hits &= hits - 1;
       const uint64_t ct = base + k * nwaves;
-      // every plane and tail bit-plane of the tile in flight together
-      uint4 wp[kMaxPlanes];
-      uint32_t th[7];
-#pragma unroll
-      for (uint32_t p = 0; p < kMaxPlanes; ++p) wp[p] = p < cv.P ? load_plane(cv, p, ct, lane) : make_uint4(0, 0, 0, 0);
-#pragma unroll
-      for (uint32_t j = 0; j < 7; ++j) th[j] = j < cv.r ? load_tail(cv, j, ct, lane) : 0u;
-      uint64_t off[16];
-#pragma unroll
-      for (uint32_t b = 0; b < 16; ++b) off[b] = 0;
-#pragma unroll
-      for (uint32_t p = 0; p < kMaxPlanes; ++p) {
-        if (p < cv.P) {
-#pragma unroll
-          for (uint32_t b = 0; b < 16; ++b) off[b] = (off[b] << 8) | byte_at(wp[p], b);
-        }
-      }
-#pragma unroll
-      for (int j = 6; j >= 0; --j) {
-        if ((uint32_t)j < cv.r) {
-#pragma unroll
-          for (uint32_t b = 0; b < 16; ++b) off[b] = (off[b] << 1) | ((th[j] >> b) & 1u);
-        }
-      }
-      uint64_t m = 0;
-#pragma unroll
-      for (uint32_t b = 0; b < 16; ++b) m = off[b] > m ? off[b] : m;   // rows >= n are zero
-      m = uniform_u64(wave_max_u64(m));
+      const uint64_t m = lane_max_offset(cv, ct, lane);
       best = m > best ? m : best;
       have = true;
     }
@@ -721,6 +694,7 @@ __global__ __launch_bounds__(256) void k_max_refine(ChunkView cv, const uint8_t*
   // one update per workgroup, and only while it raises the result: device
   // atomics on one address serialize (about 11 ns each)
   __shared__ unsigned long long wbest[4];
+  best = wave_max_u64(best);
   if (lane == 0) wbest[wave_in_wg()] = have ? best + 1 : 0;
   __syncthreads();
   if (threadIdx.x == 0) {
