@@ -769,7 +769,7 @@ __device__ __forceinline__ void major_mat_item(const BatchBuffers& bb, const BQu
   #pragma unroll 1
   for (uint64_t c = it.c0; c < it.c1; ++c) {
     uint64_t v[16];
-    major_tile_offsets<SEM, S>(mv, c, lane, v);
+    major_tile_offsets<SEM, S>(mv, c, lane, reinterpret_cast<uint8_t*>(sv), v);
 #pragma unroll
     for (uint32_t b = 0; b < 16; ++b) {
       const uint64_t o = (v[b] >> drop) << drop;
@@ -804,7 +804,8 @@ __device__ __forceinline__ void major_mat_item_s(const BatchBuffers& bb, const B
 }
 
 __global__ __launch_bounds__(256) void k_bq_major_mat(const BatchBuffers* __restrict__ bbp) {
-  __shared__ double s_val[4][64 * kLdsRow];
+  __shared__ __align__(16) double s_val[4][64 * kLdsRow];   // a tile's column images, then its values
+  static_assert(sizeof(s_val[0]) >= kImageBytes, "column images fit the staging");
   const BatchBuffers bb = cload(bbp);
   const WaveSlot ws = wave_slot();
   const uint32_t lane = ws.lane;

@@ -289,7 +289,8 @@ __global__ __launch_bounds__(256) void k_major_positions(const uint16_t* __restr
 template <int SEM, int S>
 __global__ __launch_bounds__(256) void k_major_decode(MajorView mv, double inv_scale, uint32_t drop,
                                                       double* __restrict__ out) {
-  __shared__ double s_val[4][64 * kLdsRow];
+  __shared__ __align__(16) double s_val[4][64 * kLdsRow];   // a tile's column images, then its values
+  static_assert(sizeof(s_val[0]) >= kImageBytes, "column images fit the staging");
   const uint32_t lane = __lane_id();
   double* sv = s_val[wave_in_wg()];
   const uint64_t wave = wave_global();
@@ -297,7 +298,7 @@ __global__ __launch_bounds__(256) void k_major_decode(MajorView mv, double inv_s
   const ChunkView& dv = mv.dense;
   for (uint64_t c = wave; c < dv.ntiles; c += nwaves) {
     uint64_t v[16];
-    major_tile_offsets<SEM, S>(mv, c, lane, v);
+    major_tile_offsets<SEM, S>(mv, c, lane, reinterpret_cast<uint8_t*>(sv), v);
 #pragma unroll
     for (uint32_t b = 0; b < 16; ++b) {
       // SEM 1: the top F - drop bits in place; SEM 2: the top F - drop bits as an

@@ -9,6 +9,8 @@
 #include <hip/hip_runtime.h>
 #include <stddef.h>
 
+#include <type_traits>
+
 #include "buff_common.h"
 #include "buff_device.h"
 #include "buff_major.h"
@@ -298,76 +300,122 @@ __device__ __forceinline__ uint32_t packed_sum(const Packed16& pk, uint32_t m16)
   return __builtin_amdgcn_sad_u8(pk.d3 & keep(3), 0u, a);
 }
 
+// LDS bytes a wave needs for major_tile_offsets' column images.
+constexpr uint32_t kImageBytes = kMaxSparse * kTileRows;
+
 // The lane's 16 stored offsets of tile c of a buff-major chunk
 // (buff_decode_majority, buff_simd.rs:633-861): column 0 places its byte; a
 // later sparse column ORs its outlier bytes at its shift and the majority byte
 // at twice its shift, and only for rows up to its last outlier (SEM: every row
 // gets its byte once, the true offset). Then the dense planes and tail.
+//
+// A sparse column's 16 bytes per lane come from an image of the tile in `img`
+// (S * 1024 bytes of the wave's LDS, the plane layout of buff_common.h): every
+// lane writes the fill byte of its rows, then outlier k of the tile goes to
+// lane k % 64, which writes its byte over it. The offsets are assembled by byte
+// permutes from the images and planes (the dense value from its lowest byte, so
+// that the positions do not depend on the number of dense planes). The kernels
+// that call this are bound by their vector instructions: walking every lane's
+// outliers by rank and shifting each plane's byte into 64 bits took 91 us
+// (compat 106) for 33,554,432 rows of three sparse columns, two planes and two
+// tail bits, now 66 (71); the values' write and the bytes' read take 62 at the
+// copy rate.
 template <int SEM, int S, typename MV>
-__device__ __forceinline__ void major_tile_offsets(const MV& mv, uint64_t c, uint32_t lane, uint64_t (&v)[16]) {
+__device__ __forceinline__ void major_tile_offsets(const MV& mv, uint64_t c, uint32_t lane, uint8_t* img,
+                                                   uint64_t (&v)[16]) {
   constexpr int SS = S > 0 ? S : 1;
   constexpr int NPM = (int)kMaxPlanes - S > 0 ? (int)kMaxPlanes - S : 1;   // dense planes at most (F <= 64)
   const ChunkView& dv = mv.dense;
-  // every load of the tile first: masks and prefixes, dense planes and tail,
-  // then the outlier windows (they need the masks' scan)
-  uint32_t m[SS], pre[SS];
+  const uint32_t P = dv.P, r = dv.r;
+  // every load of the tile first: each lane's first outlier of every column,
+  // the dense planes (w[q]: the q-th from the lowest) and the tail
+  uint32_t p0[SS], cnt[SS], row0[SS], byte0[SS], m[SS];
 #pragma unroll
   for (int j = 0; j < S; ++j) {
-    m[j] = mv.col[j].mask16[c * 64 + lane];
-    pre[j] = mv.col[j].prefix[c];
+    p0[j] = mv.col[j].prefix[c];
+    cnt[j] = mv.col[j].prefix[c + 1] - p0[j];
+    m[j] = SEM || j == 0 ? 0u : (uint32_t)mv.col[j].mask16[c * 64 + lane];
   }
-  uint4 wp[NPM];
+  uint4 w[NPM];
 #pragma unroll
-  for (int p = 0; p < NPM; ++p) wp[p] = (uint32_t)p < dv.P ? load_plane(dv, p, c, lane) : make_uint4(0, 0, 0, 0);
+  for (int q = 0; q < NPM; ++q) w[q] = (uint32_t)q < P ? load_plane(dv, P - 1 - q, c, lane) : make_uint4(0, 0, 0, 0);
   uint32_t h[7];
 #pragma unroll
-  for (uint32_t j = 0; j < 7; ++j) h[j] = j < dv.r ? load_tail(dv, j, c, lane) : 0u;
-  uint4 ws[SS];
+  for (uint32_t j = 0; j < 7; ++j) h[j] = j < r ? load_tail(dv, j, c, lane) : 0u;
 #pragma unroll
   for (int j = 0; j < S; ++j) {
-    const uint32_t excl = wave_excl_scan_u32(__popc(m[j]), lane);
-    const Packed16 pk = m[j] ? load_packed(mv.col[j].outl, (uint64_t)pre[j] + excl) : Packed16{0, 0, 0, 0};
-    ws[j] = patch_outliers(pk, m[j], m[j], mv.col[j].major);
+    const bool has = lane < cnt[j];
+    row0[j] = has ? mv.col[j].pos[p0[j] + lane] : 0u;
+    byte0[j] = has ? mv.col[j].outl[p0[j] + lane] : 0u;
   }
-  const uint64_t row0 = c * kTileRows + 16ull * lane;
-  // one column at a time over the lane's 16 rows, each behind a wave-uniform
-  // guard (absent planes and tail bits cost no instructions); the tail bits
-  // gather in 32-bit words
+  uint4 ws[SS];
+  if constexpr (S > 0) {
 #pragma unroll
-  for (uint32_t b = 0; b < 16; ++b) v[b] = 0;
+    for (int j = 0; j < S; ++j) {
+      const uint32_t M = SEM || j == 0 ? 0x01010101u * mv.col[j].major : 0u;
+      reinterpret_cast<uint4*>(img + j * kTileRows)[lane] = make_uint4(M, M, M, M);
+    }
+    wave_lds_sync();
+    auto put = [&](int j, uint32_t row, uint32_t byte) {
+      img[j * kTileRows + (row & ~15u) + 4 * (row & 3u) + ((row >> 2) & 3u)] = (uint8_t)byte;
+    };
 #pragma unroll
-  for (int j = 0; j < S; ++j) {
-    const uint32_t sh = mv.col[j].shift;
+    for (int j = 0; j < S; ++j) {
+      if (lane < cnt[j]) put(j, row0[j], byte0[j]);
+      for (uint32_t k = lane + 64; k < cnt[j]; k += 64) put(j, mv.col[j].pos[p0[j] + k], mv.col[j].outl[p0[j] + k]);
+    }
+    wave_lds_sync();
+#pragma unroll
+    for (int j = 0; j < S; ++j) ws[j] = reinterpret_cast<const uint4*>(img + j * kTileRows)[lane];
+    wave_lds_sync();   // the images may be overwritten from here on
+  }
+  // tail byte of row 4k + i in byte k of T[i], its bits at the top
+  uint32_t T[4];
+  tail_bytes<7>(h, r, T);
+  auto dword = [](const uint4& q, uint32_t i) -> uint32_t { return i == 0 ? q.x : i == 1 ? q.y : i == 2 ? q.z : q.w; };
+  // byte m of the dense value of rows b % 4 == i: the tail byte, then the planes from the lowest
+  auto dense_src = [&](int k, uint32_t i) -> uint32_t { return k == 0 ? T[i] : k - 1 < NPM ? dword(w[k - 1 < NPM ? k - 1 : 0], i) : 0u; };
+  auto dense_rows = [&](auto npairs) {
 #pragma unroll
     for (uint32_t b = 0; b < 16; ++b) {
-      const uint64_t byte = (uint64_t)byte_at(ws[j], b) << sh;
-      if (SEM || j == 0) {
-        v[b] |= byte;
-      } else {
+      const uint32_t i = b & 3, sel = (b >> 2) | (((b >> 2) + 4) << 8) | 0x0C0C0000u;
+      uint64_t X = 0;
+#pragma unroll
+      for (int k = 0; k < decltype(npairs)::value; ++k)
+        X |= (uint64_t)__builtin_amdgcn_perm(dense_src(2 * k + 1, i), dense_src(2 * k, i), sel) << (16 * k);
+      v[b] = X >> (8u - r);
+    }
+  };
+  if (P <= 1) dense_rows(std::integral_constant<int, 1>{});
+  else if (P <= 3 || NPM <= 3) dense_rows(std::integral_constant<int, 2>{});
+  else dense_rows(std::integral_constant<int, 4>{});
+  if constexpr (S > 0) {
+    // the sparse bytes above them, column 0 the highest
+    auto sparse_src = [&](int k, uint32_t i) -> uint32_t { return k < S ? dword(ws[k < S ? S - 1 - k : 0], i) : 0u; };
+#pragma unroll
+    for (uint32_t b = 0; b < 16; ++b) {
+      const uint32_t i = b & 3, sel = (b >> 2) | (((b >> 2) + 4) << 8) | 0x0C0C0000u;
+      uint64_t X = 0;
+#pragma unroll
+      for (int k = 0; 2 * k < S; ++k)
+        X |= (uint64_t)__builtin_amdgcn_perm(sparse_src(2 * k + 1, i), sparse_src(2 * k, i), sel) << (16 * k);
+      v[b] |= X << dv.F;
+    }
+    if (!SEM) {
+      const uint64_t row0 = c * kTileRows + 16ull * lane;
+#pragma unroll
+      for (int j = 1; j < S; ++j) {
+        const uint32_t sh = mv.col[j].shift;
         const uint64_t twice = ((uint64_t)mv.col[j].major << sh) << sh;
-        const uint64_t t = ((m[j] >> b) & 1u) ? byte : twice;
-        v[b] |= row0 + b <= mv.col[j].last ? t : 0ull;
+        if (!twice) continue;
+        const uint64_t last = mv.col[j].last;   // ~0 without outliers: every row
+        const uint32_t in = last >= row0 + 15 ? 0xFFFFu : (last >= row0 ? (2u << (uint32_t)(last - row0)) - 1u : 0u);
+        const uint32_t nm = ~m[j] & in;
+#pragma unroll
+        for (uint32_t b = 0; b < 16; ++b) v[b] |= (nm >> b) & 1u ? twice : 0ull;
       }
     }
   }
-#pragma unroll
-  for (int p = 0; p < NPM; ++p) {
-    if ((uint32_t)p >= dv.P) break;
-    const uint32_t sh = dv.F - 8 * (p + 1);
-#pragma unroll
-    for (uint32_t b = 0; b < 16; ++b) v[b] |= (uint64_t)byte_at(wp[p], b) << sh;
-  }
-  uint32_t t[16];
-#pragma unroll
-  for (uint32_t b = 0; b < 16; ++b) t[b] = 0;
-#pragma unroll
-  for (uint32_t j = 0; j < 7; ++j) {
-    if (j >= dv.r) break;
-#pragma unroll
-    for (uint32_t b = 0; b < 16; ++b) t[b] |= ((h[j] >> b) & 1u) << j;
-  }
-#pragma unroll
-  for (uint32_t b = 0; b < 16; ++b) v[b] |= t[b];
 }
 
 // The first S sparse columns of a MajorView (the same layout as its prefix):

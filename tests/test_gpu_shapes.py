@@ -61,3 +61,23 @@ def test_windowed_max(ctx, decimals, rows, window):
         hit[s:e] = f[s:e] == np.repeat(want, window)[: e - s]
         assert np.array_equal(bits(words, rows), hit), (s, e)
     ch.free()
+
+
+# the decode of sparse columns: one, two and more dense planes, tiles with no outlier, a few, and more than one a lane
+@pytest.mark.parametrize("layout", ["major", "residue"])
+@pytest.mark.parametrize("decimals", [1, 2, 3, 4, 6, 8])
+@pytest.mark.parametrize("rows", [2000, 40 * TILE + 7])
+def test_sparse_decode(ctx, layout, decimals, rows):
+    rng = np.random.default_rng(5)
+    x = np.round(rng.normal(100.0, 0.5, rows), decimals)
+    # the leading rows decide which columns are sparse; later tiles hold none, few, or a third of outliers
+    share = np.where(np.arange(rows) < 2000, 0.02, (np.arange(rows) // TILE % 3) / 6.0)
+    hit = rng.random(rows) < share
+    hit[7] = True
+    x[hit] = np.round(100.0 + 10.0 ** rng.uniform(5, 7, int(hit.sum())), decimals)
+    ch = ctx.encode(x, 10 ** decimals, flags=buff_amd.BUFF_MAJORITY if layout == "major" else buff_amd.BUFF_RESIDUE)
+    info = ch.info()
+    assert info.sparse_cols > 0
+    want = fixed(x, info.dlen) / 2.0 ** info.dlen
+    assert np.array_equal(ch.materialize(flags=buff_amd.BUFF_SEMANTIC), want)
+    ch.free()
