@@ -199,17 +199,26 @@ __device__ __forceinline__ uint4 gather_byte16(const uint32_t (&W)[16], uint32_t
 // shift by r byte-aligns every plane, and each plane is a byte gather. Tail
 // bit j of the 16 rows is gathered from the low bytes (already in the plane
 // layout) by one mask per dword and a nibble merge.
-__device__ __forceinline__ void store_tile_planes(const uint64_t (&off)[16], uint32_t P, uint32_t r,
-                                                  uint8_t* planes, uint64_t pitch, uint16_t* tail, uint64_t c,
-                                                  uint32_t lane) {
-  uint32_t lo[16], hi[16], low8[16];
+struct AlignedRows {
+  uint32_t lo[16], hi[16];   // off >> r
+  uint32_t low8[16];         // off's low bits (the tail in the lowest r)
+};
+__device__ __forceinline__ void align_rows(const uint64_t (&off)[16], uint32_t r, AlignedRows& ar) {
 #pragma unroll
   for (uint32_t b = 0; b < 16; ++b) {
     const uint64_t a = off[b] >> r;
-    lo[b] = (uint32_t)a;
-    hi[b] = (uint32_t)(a >> 32);
-    low8[b] = (uint32_t)off[b];
+    ar.lo[b] = (uint32_t)a;
+    ar.hi[b] = (uint32_t)(a >> 32);
+    ar.low8[b] = (uint32_t)off[b];
   }
+}
+// Byte k of off >> r of the 16 rows, in the plane layout (k uniform).
+__device__ __forceinline__ uint4 aligned_byte(const AlignedRows& ar, uint32_t k) {
+  return k < 4 ? gather_byte16(ar.lo, k) : gather_byte16(ar.hi, k - 4);
+}
+__device__ __forceinline__ void store_tile_planes(const AlignedRows& ar, uint32_t P, uint32_t r, uint8_t* planes,
+                                                  uint64_t pitch, uint16_t* tail, uint64_t c, uint32_t lane) {
+  const auto &lo = ar.lo, &hi = ar.hi, &low8 = ar.low8;
   uint8_t* tile = planes + c * kTileRows;
   uint32_t p = 0;
 #pragma unroll 1
@@ -228,6 +237,13 @@ __device__ __forceinline__ void store_tile_planes(const uint64_t (&off)[16], uin
     const uint32_t G2 = G | (G >> 4);   // byte 0: rows 0-7, byte 2: rows 8-15
     tail[(c * r + j) * 64 + lane] = (uint16_t)__builtin_amdgcn_perm(G2, G2, 0x0C0C0200u);
   }
+}
+__device__ __forceinline__ void store_tile_planes(const uint64_t (&off)[16], uint32_t P, uint32_t r,
+                                                  uint8_t* planes, uint64_t pitch, uint16_t* tail, uint64_t c,
+                                                  uint32_t lane) {
+  AlignedRows ar;
+  align_rows(off, r, ar);
+  store_tile_planes(ar, P, r, planes, pitch, tail, c, lane);
 }
 
 // The lane's 16 rows of tile c as whole offsets (planes then r tail bits),

@@ -42,24 +42,25 @@ struct MajorView {
   uint32_t F;                    // full width
 };
 
-// Encode passes. Workgroup w owns the contiguous tiles [w*tpw, (w+1)*tpw).
-// Pass 1 writes the dense planes / tail, the outlier bitmaps, each lane's
-// outlier bytes packed into its 16-byte staging slot, and per-workgroup outlier
-// totals. A one-workgroup scan turns the totals into bases; pass 2 walks each
-// workgroup's tiles in order, writes the tile prefixes and moves the staged
-// bytes to their final place.
+// Encode passes. Workgroup w (of at most kMajorEncWgs) owns the contiguous tiles
+// [w*tpw, (w+1)*tpw). Pass 1 writes the dense planes / tail, the outlier
+// bitmaps, each tile's outlier count and its outlier bytes in row order at the
+// start of the tile's stage slot, and per-workgroup outlier totals. A scan turns
+// the totals into bases; pass 2 writes the tile prefixes, the outlier bytes at
+// their final place and their row positions.
+constexpr uint32_t kMajorEncWgs = 4096;
 struct MajorEnc {
   uint32_t S;
   uint32_t nwg;
   uint64_t tpw;
   uint32_t major[kMaxSparse];
-  uint32_t shift[kMaxSparse];
   uint16_t* mask16[kMaxSparse];
   uint32_t* counts[kMaxSparse];          // per tile
-  uint8_t* stage[kMaxSparse];            // ntiles * 1024 bytes: 16-byte slot per lane
+  uint8_t* stage[kMaxSparse];            // ntiles * 1024 bytes: a slot per tile
   uint32_t* wgsum[kMaxSparse];           // per workgroup: total, then exclusive base
   uint32_t* prefix[kMaxSparse];
   uint8_t* outl[kMaxSparse];
+  uint16_t* pos[kMaxSparse];
 };
 
 // Per-query constants: target byte of every byte column (sparse then dense,
@@ -85,10 +86,9 @@ void major_enc_geometry(uint64_t ntiles, MajorEnc* me);
 hipError_t launch_major_encode(const double* x, uint64_t n, int32_t pexp, uint32_t dlen, int64_t base,
                                const ChunkView& dense, const MajorEnc& me, hipStream_t s);
 // Workgroup totals -> bases; totals[2j] = outliers, totals[2j+1] = last outlier
-// row (UINT64_MAX if none); prefix[j][ntiles] = outliers.
+// row (UINT64_MAX if none).
 hipError_t launch_major_scan(const MajorEnc& me, uint64_t ntiles, unsigned long long* totals, hipStream_t s);
-// Pass 2: tile prefixes (per workgroup range), then the outlier bytes moved to
-// their final place (grid-stride over tiles).
+// Pass 2: tile prefixes (prefix[j][ntiles] = outliers), outlier bytes and row positions.
 hipError_t launch_major_place(const MajorEnc& me, uint64_t ntiles, hipStream_t s);
 // pos of one sparse column from its bitmap and tile prefixes.
 hipError_t launch_major_positions(const uint16_t* mask16, const uint32_t* prefix, uint64_t ntiles, uint16_t* pos,

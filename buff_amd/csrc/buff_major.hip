@@ -20,42 +20,30 @@
 namespace buffgpu {
 
 // ----------------------------------------------------------------------------
-// Encode (buff_simd.rs:451-555). Pass 1 reads the float64 column once and, per
-// sparse column, stores each lane's outlier bytes packed into its own 16-byte
-// slot (one aligned store) next to the outlier bitmap; per-workgroup outlier
-// totals come from per-lane popcounts. The one-workgroup scan makes the totals
-// bases (and finds the last outlier row); pass 2 walks each workgroup's tiles in
-// order and moves the packed bytes to their place in the compacted array.
-
-__device__ __forceinline__ void pack_outliers(const uint64_t (&off)[16], uint32_t sh, uint32_t m, uint64_t& lo,
-                                              uint64_t& hi) {
-  lo = 0;
-  hi = 0;
-  uint32_t k = 0;
-#pragma unroll
-  for (uint32_t b = 0; b < 16; ++b) {
-    const uint64_t v = (off[b] >> sh) & 0xFF;
-    if ((m >> b) & 1u) {
-      if (k < 8) lo |= v << (8 * k);
-      else hi |= v << (8 * (k - 8));
-      ++k;
-    }
-  }
-}
+// Encode (buff_simd.rs:451-555). Pass 1 reads the float64 column once and
+// writes the dense planes and, per sparse column, the outlier bitmap and the
+// tile's outlier bytes in row order at the start of the tile's 1024-byte stage
+// slot (so pass 2 reads one or two lines of it); per-workgroup totals come from
+// the tiles' counts. The scan makes the totals bases (and finds the last outlier
+// row); pass 2 derives each tile's prefix from its workgroup's base and counts,
+// and writes prefixes, outlier bytes and row positions. (With a 16-byte stage
+// slot per lane, a one-workgroup scan and pass 2 as four kernels, 33,554,432
+// rows with three sparse columns of 5% outliers took 92 + 27 + 55 us; now
+// 76 + 5 + 21.)
 
 __global__ __launch_bounds__(256) void k_major_encode(const double* __restrict__ x, uint64_t n, uint64_t ntiles,
                                                       int32_t pexp, uint32_t dlen, int64_t base, ChunkView dense,
                                                       MajorEnc me) {
-  __shared__ uint64_t s_off[4][64 * kLdsRow];
+  __shared__ __align__(16) uint64_t s_off[4][64 * kLdsRow];   // a tile's offsets, then its outlier bytes per column
+  static_assert(sizeof(s_off[0]) >= kMaxSparse * kTileRows, "outlier bytes fit the staging");
   __shared__ uint32_t s_cnt[kMaxSparse][4];
   const uint32_t lane = __lane_id();
   const uint32_t wslot = wave_in_wg();
   uint64_t* so = s_off[wslot];
+  uint8_t* sb = reinterpret_cast<uint8_t*>(so);
   const uint64_t t0 = (uint64_t)blockIdx.x * me.tpw;
   const uint64_t t1 = min(t0 + me.tpw, ntiles);
-  uint32_t lcnt[kMaxSparse];
-#pragma unroll
-  for (uint32_t j = 0; j < kMaxSparse; ++j) lcnt[j] = 0;
+  uint32_t total = 0;   // lane j: this wave's outliers of column j
   for (uint64_t c = t0 + wslot; c < t1; c += 4) {
     uint64_t v[16];
     const bool full = tile_full(n, c);
@@ -71,34 +59,35 @@ __global__ __launch_bounds__(256) void k_major_encode(const double* __restrict__
     for (uint32_t b = 0; b < 16; ++b) off[b] = so[kLdsRow * lane + b];
     wave_lds_sync();
     const uint32_t valid = lane_valid16(n, c, lane);
-    store_tile_planes(off, dense.P, dense.r, dense.planes, dense.pitch, dense.tail, c, lane);
+    AlignedRows ar;
+    align_rows(off, dense.r, ar);
+    store_tile_planes(ar, dense.P, dense.r, dense.planes, dense.pitch, dense.tail, c, lane);
+    uint32_t tile_cnt = 0;   // lane j: the tile's outliers of column j
 #pragma unroll 1
     for (uint32_t j = 0; j < me.S; ++j) {
-      const uint32_t sh = me.shift[j], mj = me.major[j];
-      uint32_t m = 0;
-#pragma unroll
-      for (uint32_t b = 0; b < 16; ++b) m |= (uint32_t)(((off[b] >> sh) & 0xFF) != mj) << b;
-      m &= valid;
+      // column j's byte is byte P + S - 1 - j of off >> r
+      const uint4 w = aligned_byte(ar, dense.P + me.S - 1 - j);
+      const uint32_t m = ~mask_eq(w, make_digit(me.major[j])) & valid;
       me.mask16[j][c * 64 + lane] = (uint16_t)m;
-      const uint32_t tile_cnt = wave_total_u32(__popc(m));
-      if (lane == 0) me.counts[j][c] = tile_cnt;
-      if (m) {
-        uint64_t lo, hi;
-        pack_outliers(off, sh, m, lo, hi);
-        reinterpret_cast<uint4*>(me.stage[j] + c * kTileRows)[lane] =
-            make_uint4((uint32_t)lo, (uint32_t)(lo >> 32), (uint32_t)hi, (uint32_t)(hi >> 32));
-      }
       const uint32_t pc = __popc(m);
-#pragma unroll
-      for (uint32_t jj = 0; jj < kMaxSparse; ++jj) lcnt[jj] += jj == j ? pc : 0u;   // registers, not scratch
+      const uint32_t excl = wave_excl_scan_u32(pc, lane);
+      const uint32_t cnt = (uint32_t)__builtin_amdgcn_readlane((int)(excl + pc), 63);
+      if (lane == j) tile_cnt = cnt;
+      uint8_t* at = sb + j * kTileRows + excl;
+      for (uint32_t rem = m; rem; rem &= rem - 1u) *at++ = (uint8_t)byte_at(w, (uint32_t)__builtin_ctz(rem));
     }
+    wave_lds_sync();
+#pragma unroll 1
+    for (uint32_t j = 0; j < me.S; ++j) {
+      const uint32_t cnt = (uint32_t)__builtin_amdgcn_readlane((int)tile_cnt, j);
+      if (lane == 0) me.counts[j][c] = cnt;
+      uint32_t* dst = reinterpret_cast<uint32_t*>(me.stage[j] + c * kTileRows);
+      for (uint32_t i = lane; 4 * i < cnt; i += 64) dst[i] = reinterpret_cast<const uint32_t*>(sb + j * kTileRows)[i];
+    }
+    wave_lds_sync();
+    total += tile_cnt;
   }
-#pragma unroll
-  for (uint32_t j = 0; j < kMaxSparse; ++j) {
-    if (j >= me.S) break;
-    const uint32_t w = wave_sum_u32(lcnt[j]);
-    if (lane == 0) s_cnt[j][wslot] = w;
-  }
+  if (lane < me.S) s_cnt[lane][wslot] = total;
   __syncthreads();
   if (threadIdx.x < me.S) {
     const uint32_t j = threadIdx.x;
@@ -106,116 +95,93 @@ __global__ __launch_bounds__(256) void k_major_encode(const double* __restrict__
   }
 }
 
-// One workgroup: per column, the workgroup totals become exclusive bases, and
-// the last outlier row is found in the last workgroup range holding outliers.
-__global__ __launch_bounds__(256) void k_major_scan(MajorEnc me, uint64_t ntiles,
-                                                    unsigned long long* __restrict__ totals) {
-  __shared__ uint32_t s_sum[256];
-  __shared__ int32_t s_lastwg[256];
-  __shared__ unsigned long long s_row[256];
-  const uint32_t tid = threadIdx.x;
-  const uint32_t per = (me.nwg + 255) / 256;
-  for (uint32_t j = 0; j < me.S; ++j) {
-    uint32_t* ws = me.wgsum[j];
-    const uint32_t a0 = min(tid * per, me.nwg), a1 = min(a0 + per, me.nwg);
-    uint32_t local = 0;
-    int32_t lastwg = -1;
-    for (uint32_t i = a0; i < a1; ++i) {
-      const uint32_t k = ws[i];
-      local += k;
-      if (k) lastwg = (int32_t)i;
+// One workgroup per column: its workgroup totals (at most kMajorEncWgs) become
+// exclusive bases, and the last outlier row is found in the last workgroup
+// range holding outliers.
+__global__ __launch_bounds__(1024) void k_major_scan(MajorEnc me, uint64_t ntiles,
+                                                     unsigned long long* __restrict__ totals) {
+  constexpr uint32_t kPer = kMajorEncWgs / 1024;
+  __shared__ uint32_t s_wave[16], s_last[16];
+  __shared__ unsigned long long s_row[16];
+  const uint32_t tid = threadIdx.x, lane = __lane_id(), wave = wave_in_wg();
+  const uint32_t j = blockIdx.x;
+  uint32_t* ws = me.wgsum[j];
+  uint32_t k[kPer], sum = 0, last = 0;   // last: index + 1 of the last range with outliers
+#pragma unroll
+  for (uint32_t q = 0; q < kPer; ++q) {
+    const uint32_t i = tid * kPer + q;
+    k[q] = i < me.nwg ? ws[i] : 0u;
+    sum += k[q];
+    if (k[q]) last = i + 1;
+  }
+  const uint32_t excl = wave_excl_scan_u32(sum, lane);
+  last = wave_max_u32_dpp(last);
+  if (lane == 63) s_wave[wave] = excl + sum;
+  if (lane == 0) s_last[wave] = last;
+  __syncthreads();
+  uint32_t run = excl, total = 0;
+  last = 0;
+#pragma unroll
+  for (uint32_t w = 0; w < 16; ++w) {
+    run += w < wave ? s_wave[w] : 0u;
+    total += s_wave[w];
+    last = max(last, s_last[w]);
+  }
+#pragma unroll
+  for (uint32_t q = 0; q < kPer; ++q) {
+    const uint32_t i = tid * kPer + q;
+    if (i < me.nwg) ws[i] = run;
+    run += k[q];
+  }
+  // last outlier row: highest set bit in the masks of that range's tiles
+  unsigned long long best = 0;   // row + 1
+  if (last) {
+    const uint64_t w0 = (uint64_t)(last - 1) * me.tpw * 64;
+    const uint64_t w1 = min((uint64_t)last * me.tpw, ntiles) * 64;
+    for (uint64_t w = w0 + tid; w < w1; w += 1024) {
+      const uint32_t m = me.mask16[j][w];
+      if (m) best = max(best, (unsigned long long)(16 * w + (32u - (uint32_t)__clz(m))));
     }
-    s_sum[tid] = local;
-    s_lastwg[tid] = lastwg;
-    __syncthreads();
-    for (uint32_t o = 1; o < 256; o <<= 1) {
-      const uint32_t a = tid >= o ? s_sum[tid - o] : 0u;
-      __syncthreads();
-      s_sum[tid] += a;
-      __syncthreads();
-    }
-    for (uint32_t o = 128; o > 0; o >>= 1) {
-      if (tid < o) s_lastwg[tid] = max(s_lastwg[tid], s_lastwg[tid + o]);
-      __syncthreads();
-    }
-    uint32_t run = s_sum[tid] - local;
-    for (uint32_t i = a0; i < a1; ++i) {
-      const uint32_t k = ws[i];
-      ws[i] = run;
-      run += k;
-    }
-    // last outlier row: highest set bit in the masks of that workgroup's tiles
-    const int32_t lw = s_lastwg[0];
-    unsigned long long best = 0;   // row + 1
-    if (lw >= 0) {
-      const uint64_t w0 = (uint64_t)lw * me.tpw * 64;
-      const uint64_t w1 = min(((uint64_t)lw + 1) * me.tpw, ntiles) * 64;
-      for (uint64_t w = w0 + tid; w < w1; w += 256) {
-        const uint32_t m = me.mask16[j][w];
-        if (m) best = max(best, (unsigned long long)(16 * w + (32u - (uint32_t)__clz(m))));
-      }
-    }
-    s_row[tid] = best;
-    __syncthreads();
-    for (uint32_t o = 128; o > 0; o >>= 1) {
-      if (tid < o) s_row[tid] = max(s_row[tid], s_row[tid + o]);
-      __syncthreads();
-    }
-    if (tid == 0) {
-      const uint32_t total = s_sum[255];
-      me.prefix[j][ntiles] = total;
-      totals[2 * j] = total;
-      totals[2 * j + 1] = s_row[0] ? s_row[0] - 1 : ~0ull;
-    }
-    __syncthreads();
+  }
+  best = wave_max_u64(best);
+  if (lane == 0) s_row[wave] = best;
+  __syncthreads();
+  if (tid == 0) {
+    for (uint32_t w = 1; w < 16; ++w) best = max(best, s_row[w]);
+    totals[2 * j] = total;
+    totals[2 * j + 1] = best ? best - 1 : ~0ull;
   }
 }
 
-// Pass 2a: workgroup w scans the counts of its tiles (256 at a time) from its base.
-__global__ __launch_bounds__(256) void k_major_tileprefix(MajorEnc me, uint64_t ntiles) {
-  __shared__ uint32_t s_sum[256];
-  const uint32_t tid = threadIdx.x;
+// Pass 2: the tiles of pass 1's workgroup range. Every wave scans the counts of
+// the range's tiles (64 at a time) from its base, and takes every fourth tile:
+// the outlier bytes move from the stage slot to their place, the row positions
+// come from the bitmap.
+__global__ __launch_bounds__(256) void k_major_place(MajorEnc me, uint64_t ntiles) {
+  const uint32_t lane = __lane_id(), wave = wave_in_wg();
   const uint64_t t0 = (uint64_t)blockIdx.x * me.tpw;
   const uint64_t t1 = min(t0 + me.tpw, ntiles);
+#pragma unroll 1
   for (uint32_t j = 0; j < me.S; ++j) {
     uint32_t carry = me.wgsum[j][blockIdx.x];
-    for (uint64_t g = t0; g < t1; g += 256) {
-      const uint64_t c = g + tid;
-      const uint32_t cnt = c < t1 ? me.counts[j][c] : 0u;
-      s_sum[tid] = cnt;
-      __syncthreads();
-      for (uint32_t o = 1; o < 256; o <<= 1) {
-        const uint32_t a = tid >= o ? s_sum[tid - o] : 0u;
-        __syncthreads();
-        s_sum[tid] += a;
-        __syncthreads();
-      }
-      if (c < t1) me.prefix[j][c] = carry + s_sum[tid] - cnt;
-      carry += s_sum[255];
-      __syncthreads();
-    }
-  }
-}
-
-// Pass 2b: every tile's staged outlier bytes to prefix[c] + lane offset.
-__global__ __launch_bounds__(256) void k_major_copy(MajorEnc me, uint64_t ntiles) {
-  const uint32_t lane = __lane_id();
-  const uint64_t wave = wave_global();
-  const uint64_t nwaves = waves_in_grid();
-  for (uint64_t c = wave; c < ntiles; c += nwaves) {
-#pragma unroll 1
-    for (uint32_t j = 0; j < me.S; ++j) {
-      const uint32_t m = me.mask16[j][c * 64 + lane];
-      const uint32_t pre = me.prefix[j][c];
-      const uint32_t pc = __popc(m);
-      const uint32_t excl = wave_excl_scan_u32(pc, lane);
-      if (m) {
-        const uint4 w = reinterpret_cast<const uint4*>(me.stage[j] + c * kTileRows)[lane];
-        const uint64_t lo = (uint64_t)w.x | ((uint64_t)w.y << 32), hi = (uint64_t)w.z | ((uint64_t)w.w << 32);
-        uint8_t* dst = me.outl[j] + pre + excl;
-        for (uint32_t k = 0; k < pc; ++k) dst[k] = (uint8_t)(((k < 8 ? lo : hi) >> (8 * (k & 7))) & 0xFF);
+    for (uint64_t g = t0; g < t1; g += 64) {
+      const uint64_t cl = g + lane;
+      const uint32_t cnt = cl < t1 ? me.counts[j][cl] : 0u;
+      const uint32_t pre = carry + wave_excl_scan_u32(cnt, lane);
+      if (wave == 0 && cl < t1) me.prefix[j][cl] = pre;
+      carry = (uint32_t)__builtin_amdgcn_readlane((int)(pre + cnt), 63);
+      const uint32_t in = (uint32_t)min((uint64_t)64, t1 - g);
+      for (uint32_t u = wave; u < in; u += 4) {
+        const uint64_t c = g + u;
+        const uint32_t p0 = (uint32_t)__builtin_amdgcn_readlane((int)pre, u);
+        const uint32_t k = (uint32_t)__builtin_amdgcn_readlane((int)cnt, u);
+        uint32_t m = me.mask16[j][c * 64 + lane];
+        for (uint32_t i = lane; i < k; i += 64) me.outl[j][p0 + i] = me.stage[j][c * kTileRows + i];
+        uint16_t* at = me.pos[j] + p0 + wave_excl_scan_u32(__popc(m), lane);
+        for (; m; m &= m - 1u) *at++ = (uint16_t)(16 * lane + (uint32_t)__builtin_ctz(m));
       }
     }
+    if (blockIdx.x == gridDim.x - 1 && threadIdx.x == 0) me.prefix[j][ntiles] = carry;
   }
 }
 
@@ -794,7 +760,7 @@ static inline uint32_t tiles_grid(uint64_t ntiles, uint32_t max_wg) {
 
 void major_enc_geometry(uint64_t ntiles, MajorEnc* me) {
   uint64_t nwg = (ntiles + 3) / 4;
-  if (nwg > 4096) nwg = 4096;
+  if (nwg > kMajorEncWgs) nwg = kMajorEncWgs;
   if (nwg < 1) nwg = 1;
   me->tpw = (ntiles + nwg - 1) / nwg;
   me->nwg = (uint32_t)((ntiles + me->tpw - 1) / me->tpw);
@@ -809,15 +775,13 @@ hipError_t launch_major_encode(const double* x, uint64_t n, int32_t pexp, uint32
 }
 
 hipError_t launch_major_scan(const MajorEnc& me, uint64_t ntiles, unsigned long long* totals, hipStream_t s) {
-  launch_k(k_major_scan, dim3(1), dim3(256), 0, s, me, ntiles, totals);
+  if (me.nwg > kMajorEncWgs) return hipErrorInvalidValue;
+  launch_k(k_major_scan, dim3(me.S), dim3(1024), 0, s, me, ntiles, totals);
   return hipGetLastError();
 }
 
 hipError_t launch_major_place(const MajorEnc& me, uint64_t ntiles, hipStream_t s) {
-  launch_k(k_major_tileprefix, dim3(me.nwg), dim3(256), 0, s, me, ntiles);
-  hipError_t e = hipGetLastError();
-  if (e != hipSuccess) return e;
-  launch_k(k_major_copy, dim3(tiles_grid(ntiles, 4096)), dim3(256), 0, s, me, ntiles);
+  launch_k(k_major_place, dim3(me.nwg), dim3(256), 0, s, me, ntiles);
   return hipGetLastError();
 }
 

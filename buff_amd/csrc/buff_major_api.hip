@@ -118,10 +118,10 @@ MajorEnc enc_of(const Chunk* ch, uint8_t* scratch) {
   const EncScratch l = enc_layout(ch->S, ch->view.ntiles, me.nwg);
   for (uint32_t j = 0; j < ch->S; ++j) {
     me.major[j] = ch->sp[j].major;
-    me.shift[j] = ch->sp[j].shift;
     me.mask16[j] = ch->sp[j].mask16;
     me.prefix[j] = ch->sp[j].prefix;
     me.outl[j] = ch->sp[j].outl;
+    me.pos[j] = ch->sp[j].pos;
     if (scratch) {
       me.stage[j] = scratch + l.stage + (uint64_t)j * ch->view.ntiles * kTileRows;
       me.counts[j] = (uint32_t*)(scratch + l.counts) + (uint64_t)j * ch->view.ntiles;
@@ -350,7 +350,6 @@ int major_build(Ctx* ctx, const double* x, uint64_t n, uint64_t scale, uint32_t 
   {
     ProfScope ps(ctx, "k_major_place");
     e = launch_major_place(me, ch->view.ntiles, ctx->stream);
-    if (e == hipSuccess) e = build_positions(ctx, ch);
   }
   if (e != hipSuccess) {
     free_partial(ctx, ch);
