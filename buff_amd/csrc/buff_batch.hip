@@ -659,12 +659,13 @@ __device__ __forceinline__ uint32_t major_filter_item(const MajorPrefix<S>& mv, 
 #pragma unroll
   for (uint32_t k = 0; k < kMaxPlanes; ++k) tg.digit[k] = q.tg.digit[k];
   tg.tail = q.tg.tail;
+  const MajorRules<S> ru = major_rules<MODE, S>(mv, tg, sem);
   uint32_t count = 0;
   // two tiles in flight per step (the second may lie past the item: computed, not stored)
   #pragma unroll 1
   for (uint64_t c = it.c0; c < it.c1; c += 2) {
     uint32_t res[2];
-    major_filter_group<MODE, S, 2>(mv, tg, sem, c, lane, dep, res);
+    major_filter_group<MODE, S, 2>(mv, tg, ru, c, lane, dep, res);
     filter_store<MODE>(mv.dense, out16, c, lane, res[0], count);
     if (c + 1 < it.c1) filter_store<MODE>(mv.dense, out16, c + 1, lane, res[1], count);
   }
@@ -737,7 +738,7 @@ __device__ __forceinline__ void major_scan_item(const BatchBuffers& bb, const BQ
 }
 
 __global__ __launch_bounds__(256) void k_bq_major(const BatchBuffers* __restrict__ bbp) {
-  __shared__ unsigned long long s_dep[4][64];
+  __shared__ unsigned long long s_dep[4][dep_words(7, 2)];
   const BatchBuffers bb = cload(bbp);
   const WaveSlot ws = wave_slot();
   const uint32_t lane = ws.lane;

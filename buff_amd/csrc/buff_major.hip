@@ -202,9 +202,9 @@ __global__ __launch_bounds__(256) void k_major_place(MajorEnc me, uint64_t ntile
 // candidates' later planes and tail. S (sparse columns) is a template argument so
 // the per-column state stays in registers.
 template <int MODE, int S, int U, bool PF>
-__global__ __launch_bounds__(256) void k_major_filter(MajorView mv, MajorTarget tg, uint32_t sem,
+__global__ __launch_bounds__(256) void k_major_filter(MajorPrefix<S> mv, MajorTarget tg, uint32_t sem,
                                                       uint64_t* __restrict__ out, uint64_t nwords) {
-  __shared__ unsigned long long s_dep[4][64];
+  __shared__ unsigned long long s_dep[4][dep_words(S, U)];
   unsigned long long* dep = s_dep[wave_in_wg()];
   const uint32_t lane = __lane_id();
   const uint64_t wave = wave_global();
@@ -213,10 +213,11 @@ __global__ __launch_bounds__(256) void k_major_filter(MajorView mv, MajorTarget 
   uint16_t* out16 = reinterpret_cast<uint16_t*>(out);
   const uint64_t nout16 = 4 * nwords;
   const uint64_t ngroups = (dv.ntiles + U - 1) / U;
+  const MajorRules<S> ru = major_rules<MODE, S>(mv, tg, sem != 0);
   for (uint64_t grp = wave; grp < ngroups; grp += nwaves) {
     const uint64_t c0 = grp * U;
     uint32_t res[U];
-    major_filter_group<MODE, S, U, PF>(mv, tg, sem != 0, c0, lane, dep, res);
+    major_filter_group<MODE, S, U, PF>(mv, tg, ru, c0, lane, dep, res);
 #pragma unroll
     for (int u = 0; u < U; ++u) {
       const uint64_t c = c0 + u;
@@ -811,7 +812,10 @@ static void launch_filter_pf(const MajorView& mv, bool semantic, const MajorTarg
   const uint64_t groups = (mv.dense.ntiles + U - 1) / U;
   static const uint32_t fit = resident_wgs(k_major_filter<MODE, S, U, PF>);   // once per kernel
   const uint32_t grid = tiles_grid(groups, fit ? std::min(max_wg, fit) : max_wg);
-  launch_k((k_major_filter<MODE, S, U, PF>), dim3(grid), dim3(256), 0, s, mv, tg, semantic ? 1u : 0u, out, nwords);
+  MajorPrefix<S> pv;   // the columns in use only: a kernel argument lives in scalar registers
+  pv.dense = mv.dense;
+  for (int j = 0; j < S; ++j) pv.col[j] = mv.col[j];
+  launch_k((k_major_filter<MODE, S, U, PF>), dim3(grid), dim3(256), 0, s, pv, tg, semantic ? 1u : 0u, out, nwords);
 }
 
 template <int MODE, int S>

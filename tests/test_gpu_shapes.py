@@ -6,6 +6,7 @@ import pytest
 
 import buff_amd
 from buff_amd import datagen
+from oracle import refcpu
 
 pytestmark = pytest.mark.gpu
 
@@ -80,4 +81,30 @@ def test_sparse_decode(ctx, layout, decimals, rows):
     assert info.sparse_cols > 0
     want = fixed(x, info.dlen) / 2.0 ** info.dlen
     assert np.array_equal(ch.materialize(flags=buff_amd.BUFF_SEMANTIC), want)
+    ch.free()
+
+
+# the filter of sparse columns: up to three columns deposited together, then more; predicates on a majority value (the
+# dense planes are prefetched), an outlier value, and beyond the column
+@pytest.mark.parametrize("decimals", [3, 6, 8, 10])
+@pytest.mark.parametrize("rows", [2000, 3 * TILE, 41 * TILE + 5])
+def test_sparse_filter(ctx, decimals, rows):
+    rng = np.random.default_rng(6)
+    x = np.round(rng.normal(100.0, 0.001, rows), decimals)
+    hit = rng.random(rows) < 0.1
+    hit[:2] = True
+    x[hit] = np.round(10.0 ** rng.uniform(2, 5, int(hit.sum())), decimals)
+    x[1] = 0.0
+    ch = ctx.encode(x, 10 ** decimals, flags=buff_amd.BUFF_MAJORITY)
+    stream = refcpu.major_encode(x, 10 ** decimals)
+    info = ch.info()
+    f = fixed(x, info.dlen)
+    for pred in (float(x[~hit][3]), 100.0, float(x[hit][5]), 0.0, -1.0, 2e5):
+        p = int(fixed(pred, info.dlen))
+        for op, want in (("range", f > p), ("equal", f == p)):
+            words, count = ch.filter(op, pred, flags=buff_amd.BUFF_SEMANTIC)
+            assert np.array_equal(bits(words, rows), want) and count == want.sum(), (op, pred, info.sparse_cols)
+            words, count = ch.filter(op, pred)
+            w_ref, c_ref = refcpu.major_filter(stream, 10 ** decimals, op, pred)[:2]
+            assert count == c_ref and np.array_equal(words, w_ref), (op, pred, info.sparse_cols)
     ch.free()
