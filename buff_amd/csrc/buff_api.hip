@@ -312,7 +312,39 @@ int Ctx::prof_collect() {
 LaunchShape Ctx::shape(Op op, const ChunkView& v) const {
   auto it = tuned.find(tune_key(op, v.ntiles, v.P));
   if (it != tuned.end()) return it->second;
-  return LaunchShape{4, 0, 0};
+  return default_shape(op, v.ntiles);
+}
+
+// The shape of an operation that was not tuned, by the column's tiles (times:
+// kernels of walk and uniform columns, as the tuner and a trace give them).
+LaunchShape default_shape(Op op, uint64_t ntiles) {
+  switch (op) {
+    case Op::FilterGt:
+    case Op::FilterEq:
+      // Few tiles: two per wave instead of four, so that more waves share them
+      // and refine fewer tiles in turn, and the next tiles' plane loaded before
+      // the refinement (1M rows 6.7 -> 5.0 us, cold 7.7 -> 4.8; 4M cold 8.0 -> 5.7).
+      if (ntiles <= 8192) return LaunchShape{2, 2048, 2, 1};
+      // Many: a group of four tiles a wave, the workgroups beyond the resident
+      // ones started as others end, instead of resident ones that loop and wait
+      // for the slowest (134M rows, walk 31.6 -> 26.5, uniform cold 48.0 ->
+      // 42.3; 67M 20.3 -> 18.2). At 17M the resident grid is as fast.
+      if (ntiles > 32768) return LaunchShape{2, 16384, 4, 0};
+      return LaunchShape{4, 0, 0, 0};
+    case Op::Encode:
+    case Op::Materialize:
+      // the same (materialize: 17M rows 33.4 -> 32.1 us, 67M cold 141 -> 125,
+      // 134M cold 287 -> 266; encode: 17M 32.4 -> 31.4, 67M 133 -> 120)
+      return LaunchShape{4, 16384, 0, 0};
+    case Op::Sum:
+      // few tiles: one per wave (1M rows 4.8 -> 4.1 us); many: half the
+      // resident waves, whose own loads keep memory busy (134M cold 79.6 -> 70.5)
+      if (ntiles <= 4096) return LaunchShape{4, 1024, 1, 0};
+      if (ntiles <= 32768) return LaunchShape{4, 1024, 2, 0};
+      return LaunchShape{2, 1024, 2, 0};
+    default:
+      return LaunchShape{4, 0, 0, 0};
+  }
 }
 
 uint32_t tune_bucket(uint64_t ntiles) {

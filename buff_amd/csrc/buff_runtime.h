@@ -47,6 +47,8 @@ inline uint64_t tune_key(Op op, uint64_t ntiles, uint32_t planes) {
   return ((uint64_t)op << 40) | ((uint64_t)planes << 32) | tune_bucket(ntiles);
 }
 
+LaunchShape default_shape(Op op, uint64_t ntiles);
+
 struct Scratch {
   void* ptr = nullptr;
   uint64_t bytes = 0;
