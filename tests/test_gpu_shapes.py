@@ -6,7 +6,7 @@ import pytest
 
 import buff_amd
 from buff_amd import datagen
-from oracle import refcpu
+from oracle import refcpu, refcsv
 
 pytestmark = pytest.mark.gpu
 
@@ -108,3 +108,34 @@ def test_sparse_filter(ctx, decimals, rows):
             w_ref, c_ref = refcpu.major_filter(stream, 10 ** decimals, op, pred)[:2]
             assert count == c_ref and np.array_equal(words, w_ref), (op, pred, info.sparse_cols)
     ch.free()
+
+
+# short decimals (up to 8 digits, a point, up to 8 digits: the byte-parallel parse), the forms next to them, forms that
+# are none, and every item position relative to a 4 KiB block; more blocks than one round of the scan
+@pytest.mark.parametrize("skip", [0, 2])
+@pytest.mark.parametrize("seed,count,line", [(1, 3, 3), (2, 5000, 7), (3, 40_000, 1000), (4, 40_000, 10 ** 9)])
+def test_csv_short_decimals(ctx, skip, seed, count, line):
+    rng = np.random.default_rng(seed)
+    items = []
+    for _ in range(count):
+        a = "".join(rng.choice(list("0123456789"), rng.integers(0, 11)))
+        b = "".join(rng.choice(list("0123456789"), rng.integers(0, 11)))
+        form = rng.integers(0, 12)
+        s = {0: a, 1: "." + b, 2: a + ".", 3: a + "." + b + "e3", 4: a + ".." + b, 5: a + "x" + b}.get(form, a + "." + b)
+        items.append(("", "", "-", "+")[rng.integers(0, 4)] + s)
+    text = "".join(t + (("\r\n" if i % 3 else "\n") if (i + 1) % line == 0 else ",") for i, t in enumerate(items))
+    for tail in ("", "7.25", "\n"):
+        t = (text + tail).encode()
+        got = ctx.csv_parse(t, b",", skip)
+        want = np.array(refcsv.construct_file_iterator_skip_newline(t, skip), dtype=np.float64)
+        assert np.array_equal(got.view(np.uint64), want.view(np.uint64))
+
+
+def test_csv_many_blocks(ctx):
+    k = np.arange(4_500_000, dtype=np.int64) % 9973 * 1009   # 8193 blocks and more
+    body = np.char.zfill(k.astype("U8"), 8)
+    text = np.full((len(k), 9), ord(","), dtype=np.uint8)
+    text[:, :8] = np.frombuffer(body.astype("S8").tobytes(), dtype=np.uint8).reshape(-1, 8)
+    text[99::100, 8] = ord("\n")
+    assert np.array_equal(ctx.csv_parse(text.tobytes()), k.astype(np.float64))
+    assert np.array_equal(ctx.csv_parse(text.tobytes(), skip_val=3), k.reshape(-1, 100)[:, 3:].ravel().astype(np.float64))
