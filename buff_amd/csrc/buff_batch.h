@@ -120,7 +120,7 @@ constexpr uint32_t kMatGrid = 1024;
 
 constexpr uint64_t kHostQueries = 256;   // byte offset of the queries in host_in
 
-// Kernels a batch needs: the scan (filters, sums, maxima and their fold), the
+// Kernels a batch needs besides the fold: the scan (filters, sums, maxima), the
 // max refinement, the materialization, and the same for queries on buff-major
 // chunks with sparse columns (kernels of their own, so the plain kernels keep
 // their register budget).

@@ -824,11 +824,9 @@ __global__ __launch_bounds__(256) void k_bq_major_mat(const BatchBuffers* __rest
 
 hipError_t launch_batch_queries(const BatchBuffers* bb, const BatchTuning& tu, uint32_t parts, hipStream_t s) {
   hipLaunchKernelGGL(k_bq_fetch, dim3(1024), dim3(256), 0, s, bb);
-  if (parts & kBqPartScan) {
-    hipLaunchKernelGGL(k_bq_scan, dim3(tu.grid), dim3(256), 0, s, bb, tu);
-    if (parts & kBqPartMajor) hipLaunchKernelGGL(k_bq_major, dim3(tu.grid), dim3(256), 0, s, bb);
-    hipLaunchKernelGGL(k_bq_reduce, dim3(1024), dim3(256), 0, s, bb);
-  }
+  if (parts & kBqPartScan) hipLaunchKernelGGL(k_bq_scan, dim3(tu.grid), dim3(256), 0, s, bb, tu);
+  if (parts & kBqPartMajor) hipLaunchKernelGGL(k_bq_major, dim3(tu.grid), dim3(256), 0, s, bb);
+  hipLaunchKernelGGL(k_bq_reduce, dim3(1024), dim3(256), 0, s, bb);   // also the results of queries without tiles
   if (parts & kBqPartMax) {
     hipLaunchKernelGGL(k_bq_max_refine, dim3(tu.grid < 2048 ? tu.grid : 2048), dim3(256), 0, s, bb);
     hipLaunchKernelGGL(k_bq_max_publish, dim3(16), dim3(256), 0, s, bb);

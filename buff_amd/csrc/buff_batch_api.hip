@@ -318,10 +318,9 @@ int exec_reserve(QueryExec& ex, uint32_t max_q, uint64_t arena_bytes, const Batc
   BUFF_TRY(reserve(ctx, ex.arena, arena_bytes));
   BUFF_TRY(reserve(ctx, ex.bbdev, sizeof(BatchBuffers)));
   BUFF_TRY(pin_reserve(ex, max_q));
-  // every combination of kernels a batch can need (the scan always runs)
-  for (uint32_t extra = 0; extra < 16; ++extra) {
-    const uint32_t parts = kBqPartScan | ((extra & 1) ? kBqPartMax : 0u) | ((extra & 2) ? kBqPartMat : 0u) |
-                           ((extra & 4) ? kBqPartMajor : 0u) | ((extra & 8) ? kBqPartMajorMat : 0u);
+  // every combination of kernels a batch can need (maxima run in the scan)
+  for (uint32_t parts = 0; parts < 32; ++parts) {
+    if ((parts & kBqPartMax) && !(parts & kBqPartScan)) continue;
     hipGraphExec_t gx = nullptr;
     BUFF_TRY(graph_for(ex, tu, parts, &gx));
   }
@@ -504,10 +503,17 @@ int exec_launch(QueryExec& ex, const std::vector<Chunk*>& chunks, const void* vi
   // materializations are counted apart: 64 materializations of 150k rows among
   // 4096 queries made 150 items of the scans' 64 tiles, 154 us on 150 of the
   // 4096 waves.
+  // Below kItemTiles an item's own cost (its descriptors, its partial) outweighs
+  // the balance, so items get shorter only while the resident waves lack work.
+  constexpr uint64_t kResidentWaves = 8192, kItemTiles = 8;
   const uint64_t waves = 4ull * std::max<uint32_t>(tu.grid, 1);
   const uint64_t mat_waves = std::min<uint64_t>(waves, 4ull * kMatGrid);
-  const uint64_t T = std::max<uint64_t>(1, std::min<uint64_t>(Tmax, (scan_tiles + waves - 1) / waves));
-  const uint64_t Tm = std::max<uint64_t>(1, std::min<uint64_t>(Tmax, (mat_tiles + mat_waves - 1) / mat_waves));
+  auto item_tiles = [&](uint64_t tiles, uint64_t w) {
+    const uint64_t t = std::max((tiles + w - 1) / w,
+                                std::min(kItemTiles, (tiles + kResidentWaves - 1) / kResidentWaves));
+    return std::max<uint64_t>(1, std::min<uint64_t>(Tmax, t));
+  };
+  const uint64_t T = item_tiles(scan_tiles, waves), Tm = item_tiles(mat_tiles, mat_waves);
   // item ranges, by operation: sums (the longest items) first, filters, maxima
   // (whose refinement then reads only their own range), materializations;
   // k_bq_fetch writes the items on the device
@@ -576,7 +582,6 @@ int exec_launch(QueryExec& ex, const std::vector<Chunk*>& chunks, const void* vi
     else parts |= q.op == kBqMat ? kBqPartMat : kBqPartScan;
     if (q.op == kBqMax) parts |= kBqPartMax;
   }
-  parts |= kBqPartScan;   // the fold also writes the results of queries without tiles
   hipGraphExec_t gx = nullptr;
   BUFF_TRY(graph_for(ex, tu, parts, &gx));
   HIP_TRY(hipGraphLaunch(gx, ex.stream));

@@ -90,12 +90,13 @@ struct Ctx {
 
   std::map<uint64_t, LaunchShape> tuned;
   // batched queries: grid, tiles per work item, planes of the first filter pass.
-  // The grid is four times what is resident: the workgroups beyond it start as
+  // The grid is twice what is resident: the workgroups beyond it start as
   // earlier ones end, so waves whose items were short (a filter's against a
   // sum's, a chunk's last) do not wait for the others. 4096 mixed queries on
-  // 1024 chunks: 720 us on 2048 workgroups, 556 us on 8192 (536 on 16384, where
-  // 1000 maxima alone go from 108 to 130); 512 served requests 2.86 -> 2.38 ms.
-  uint32_t bt_grid = 8192, bt_tiles = 64, bt_first = 1;
+  // 1024 chunks: 720 us on 2048 workgroups, 515 on 4096, 500 on 8192; 512 served
+  // requests 2.86, 2.02 and 2.05 ms; but 47 small served ones 168, 150 and 190 us
+  // (a workgroup without an item still has to start).
+  uint32_t bt_grid = 4096, bt_tiles = 64, bt_first = 1;
   bool bt_tuned = false;
 
   ~Ctx();
