@@ -191,9 +191,15 @@ int Ctx::minmax_slots(int64_t** set, int64_t** next) {
   return BUFF_OK;
 }
 
+Publish Ctx::next_publish() {
+  Publish pub;
+  pub.mbox = mbox_dev;
+  pub.seq = ++mbox_seq;
+  return pub;
+}
+
 int Ctx::publish(const void* src, uint32_t mode, uint32_t nk, Publish* pub) {
-  pub->mbox = mbox_dev;
-  pub->seq = ++mbox_seq;
+  *pub = next_publish();
   HIP_TRY(launch_publish(src, mode, nk, *pub, stream));
   return BUFF_OK;
 }
@@ -201,10 +207,12 @@ int Ctx::publish(const void* src, uint32_t mode, uint32_t nk, Publish* pub) {
 int Ctx::published(const Publish& pub, uint64_t* words, uint32_t nw) {
   // The launch is the last work on the stream: spin on the sequence word, and
   // now and then ask the stream, so a failed launch (or one that ended
-  // without publishing) ends the wait with its error.
+  // without publishing) ends the wait with its error. A spin takes about 20 ns
+  // and asking more than 10 us: asked every 512 spins, a result that was 10 us
+  // away came 25 us later.
   for (uint32_t spin = 1;; ++spin) {
     if (__atomic_load_n(&mbox[0], __ATOMIC_ACQUIRE) == pub.seq) break;
-    if (spin % 512 == 0) {
+    if (spin % 32768 == 0) {
       const hipError_t e = hipStreamQuery(stream);
       if (e == hipSuccess) {
         if (__atomic_load_n(&mbox[0], __ATOMIC_ACQUIRE) == pub.seq) break;
@@ -224,13 +232,14 @@ int Ctx::minmax_pass(const double* x, uint64_t n, int32_t pexp, uint32_t dlen, M
   BUFF_TRY(scratch(s_partial, 3ull * nwg * sizeof(int64_t)));
   int64_t *set = nullptr, *next = nullptr;
   BUFF_TRY(minmax_slots(&set, &next));
+  Publish pub = next_publish();
+  bool fused = false;
   {
     ProfScope ps(this, "k_minmax");
-    HIP_TRY(launch_minmax_slots(x, n, pexp, dlen, (int64_t*)s_partial.ptr, set, next, nwg, stream));
-    minmax_slots_used();
+    HIP_TRY(launch_minmax_slots(x, n, pexp, dlen, (int64_t*)s_partial.ptr, set, next, nwg, stream, &pub, &fused));
+    if (!fused) minmax_slots_used();
   }
-  Publish pub;
-  BUFF_TRY(publish(set, kPublishMinMax, 0, &pub));
+  if (!fused) BUFF_TRY(publish(set, kPublishMinMax, 0, &pub));
   uint64_t w[3];
   BUFF_TRY(published(pub, w, 3));
   *mm = MinMaxOut{};
@@ -337,8 +346,11 @@ LaunchShape default_shape(Op op, uint64_t ntiles) {
       // 134M cold 287 -> 266; encode: 17M 32.4 -> 31.4, 67M 133 -> 120)
       return LaunchShape{4, 16384, 0, 0};
     case Op::Sum:
-      // few tiles: one per wave (1M rows 4.8 -> 4.1 us); many: half the
-      // resident waves, whose own loads keep memory busy (134M cold 79.6 -> 70.5)
+      // few tiles: at most 64 workgroups, which hand the sums over themselves (a
+      // call on 4097 rows 13.5 -> 11.6 us, on 1M 14.6 -> 14.0; 256 workgroups of one
+      // tile a wave 15.9), then one tile per wave; many: half the resident waves,
+      // whose own loads keep memory busy (134M cold 79.6 -> 70.5)
+      if (ntiles <= 1024) return LaunchShape{4, 64, 4, 0};
       if (ntiles <= 4096) return LaunchShape{4, 1024, 1, 0};
       if (ntiles <= 32768) return LaunchShape{4, 1024, 2, 0};
       return LaunchShape{2, 1024, 2, 0};
@@ -1029,13 +1041,14 @@ int sum_op(Ctx* ctx, const Chunk* ch, double* ref_sum, double* exact_sum, uint64
     const LaunchShape ls = ctx->shape(Op::Sum, v);
     unsigned long long *set = nullptr, *next = nullptr;
     BUFF_TRY(ctx->sum_slots(&set, &next));
+    Publish pub = ctx->next_publish();
+    bool fused = false;
     {
       ProfScope sc(ctx, "k_sum");
-      HIP_TRY(launch_sum_slots(v, set, next, ctx->stream, ls));
-      ctx->sum_slots_used();
+      HIP_TRY(launch_sum_slots(v, set, next, ctx->stream, ls, &pub, &fused));
+      if (!fused) ctx->sum_slots_used();
     }
-    Publish pub;
-    BUFF_TRY(ctx->publish(set, kPublishSumSlots, v.P + 1, &pub));
+    if (!fused) BUFF_TRY(ctx->publish(set, kPublishSumSlots, v.P + 1, &pub));
     BUFF_TRY(ctx->published(pub, ps, v.P + 1));
   }
   if (plane_sums) memcpy(plane_sums, ps, sizeof(ps));
@@ -1060,7 +1073,16 @@ int max_op(Ctx* ctx, const Chunk* ch, uint32_t flags, double* value, uint64_t* m
     return major_max(ctx, ch, flags, value, max_off, argmax);
   uint64_t best = 0;
   const ChunkView& v = ch->view;
-  if (ch->n > 0 && (v.P || v.r)) {
+  if (ch->n > 0 && (v.P || v.r) && v.ntiles <= kMaxDirectTiles) {
+    unsigned long long *set = nullptr, *next = nullptr;
+    BUFF_TRY(ctx->sum_slots(&set, &next));
+    const Publish pub = ctx->next_publish();
+    {
+      ProfScope sc(ctx, "k_max");
+      HIP_TRY(launch_max_direct(v, set, pub, ctx->stream));
+    }
+    BUFF_TRY(ctx->published(pub, &best, 1));
+  } else if (ch->n > 0 && (v.P || v.r)) {
     // [best u64 | pad to 512 | per-tile maxima]; the kernels clear best
     const uint64_t ms = max_scratch_bytes(v.ntiles);
     BUFF_TRY(ctx->scratch(ctx->s_best, 512 + ms));

@@ -49,6 +49,13 @@ enum : uint32_t {
   kPublishCopy = 2,       // nk u64 words as they are (src 8-byte aligned)
 };
 hipError_t launch_publish(const void* src, uint32_t mode, uint32_t nk, const Publish& pub, hipStream_t s);
+// A reduction of at most this many workgroups hands its result over itself: its
+// last workgroup (a ticket in the slot set) folds the slots, publishes, and
+// leaves the set empty. Every value that crosses workgroups is an agent-scope
+// atomic, so no release of the caches is needed before the ticket (with one,
+// the handover cost a large grid more than a second launch: 72 -> 160 us for a
+// sum of 134M rows); tickets of one address serialize, about 11 ns each.
+constexpr uint32_t kFusedWgs = 256;
 
 // Workgroups of the min/max pass over ntiles tiles (all resident at once).
 uint32_t minmax_grid(uint64_t ntiles);
@@ -58,11 +65,15 @@ hipError_t launch_minmax(const double* x, uint64_t n, int32_t pexp, uint32_t dle
 // into the slot set `set` (int64: kMinMaxSlots mins, kMinMaxSlots maxes, then
 // row 0's fixed value), for launch_publish to fold; `next`, the set the following
 // call folds into, is reset; `partial` gets the per-workgroup rows the
-// prefix-min pass reads. Sets start reset (launch_minmax_slots_init).
+// prefix-min pass reads. Sets start reset (launch_minmax_slots_init). With `pub`
+// and at most kFusedWgs workgroups the launch publishes the result itself
+// (*published; the set is empty again and next is as it was).
 constexpr uint32_t kMinMaxSlots = 64;
+constexpr uint32_t kMinMaxTicket = 2 * kMinMaxSlots + 1;   // word of a set
 constexpr uint32_t kMinMaxSetWords = 2 * kMinMaxSlots + 8;
 hipError_t launch_minmax_slots(const double* x, uint64_t n, int32_t pexp, uint32_t dlen, int64_t* partial,
-                               int64_t* set, int64_t* next, uint32_t nwg, hipStream_t s);
+                               int64_t* set, int64_t* next, uint32_t nwg, hipStream_t s, const Publish* pub,
+                               bool* published);
 hipError_t launch_minmax_slots_init(int64_t* sets, uint32_t nsets, hipStream_t s);
 hipError_t launch_encode(const double* x, const ChunkView& cv, int32_t pexp, hipStream_t s, const LaunchShape& ls);
 hipError_t launch_filter(const ChunkView& cv, int op, const FilterTarget& tg, uint64_t* out, uint64_t nwords,
@@ -94,11 +105,13 @@ hipError_t launch_sum(const ChunkView& cv, unsigned long long* sums, hipStream_t
 // One launch: per-plane sums (and the weighted tail sum at k = P) added into
 // the slot set `set` (u64 [kMaxPlanes + 1][kSumSlots], to be summed over the
 // slots); `next`, the set the following call adds into, is cleared. The first
-// set must be zero.
+// set must be zero. With `pub` and at most kFusedWgs workgroups the launch
+// publishes the sums itself (*published; the set is zero again).
 constexpr uint32_t kSumSlots = 64;
-constexpr uint32_t kSumSetWords = (kMaxPlanes + 1) * kSumSlots;
+constexpr uint32_t kSumTicket = (kMaxPlanes + 1) * kSumSlots;   // word of a set
+constexpr uint32_t kSumSetWords = kSumTicket + 8;
 hipError_t launch_sum_slots(const ChunkView& cv, unsigned long long* set, unsigned long long* next, hipStream_t s,
-                            const LaunchShape& ls);
+                            const LaunchShape& ls, const Publish* pub = nullptr, bool* published = nullptr);
 // Tail part of the reduced-precision sum reading q < r bits per row: out[0] +=
 // the sum of the n q-bit fields the reference reads from the packed tail,
 // out[1] += the sum of every row's top q tail bits (the caller zeroes out[0..1]).
@@ -113,6 +126,10 @@ constexpr uint32_t kMaxTagLimit = 1u << 24;
 uint64_t max_scratch_bytes(uint64_t ntiles);
 hipError_t launch_max(const ChunkView& cv, unsigned long long* best, uint8_t* scratch, unsigned int* slots,
                       uint32_t tag, hipStream_t s, const LaunchShape& ls);
+// Columns of at most kMaxDirectTiles tiles (n >= 1): one launch that rebuilds
+// every tile's offsets and publishes the max; `set`: a zero sum set, left zero.
+constexpr uint64_t kMaxDirectTiles = 4 * kFusedWgs;
+hipError_t launch_max_direct(const ChunkView& cv, unsigned long long* set, const Publish& pub, hipStream_t s);
 hipError_t launch_materialize(const ChunkView& cv, const MatParams& mp, double* out, hipStream_t s,
                               const LaunchShape& ls);
 hipError_t launch_serialize(const ChunkView& cv, uint8_t flipmask, uint8_t* body, uint64_t tail_bytes,

@@ -25,6 +25,34 @@ LaunchEvents& launch_events() {
 }
 
 // ----------------------------------------------------------------------------
+// Handing a reduction over from its own launch (kFusedWgs).
+
+// One wave: lane k < nw writes word k to the mailbox, then the sequence number
+// (a system-scope release after every lane's word).
+__device__ __forceinline__ void publish_words(const Publish& pub, uint64_t mine, uint32_t nw) {
+  const uint32_t lane = __lane_id();
+  if (lane < nw) pub.mbox[1 + lane] = mine;
+  __threadfence_system();
+  __builtin_amdgcn_wave_barrier();
+  if (lane == 0) __hip_atomic_store(pub.mbox, pub.seq, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+
+// One wave, after its slot updates (agent-scope atomics): whether its workgroup
+// is the last of the grid to get here. The wait completes the updates before the
+// ticket; the last workgroup's atomic reads then see all of them.
+__device__ __forceinline__ bool last_workgroup(unsigned long long* ticket) {
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+  uint32_t t = 0;
+  if (__lane_id() == 0)
+    t = (uint32_t)__hip_atomic_fetch_add(ticket, 1ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  return __builtin_amdgcn_readfirstlane(t) == gridDim.x - 1;
+}
+template <typename T>
+__device__ __forceinline__ T slot_load(const T* p) {
+  return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
+// ----------------------------------------------------------------------------
 // K1: fixed-point conversion + min / max reduction (encode pass 1).
 // split_double.rs:321-330. Workgroup w owns the contiguous tile range
 // [w*tpw, (w+1)*tpw), so its partial min is a segment min the prefix pass reuses.
@@ -34,7 +62,7 @@ LaunchEvents& launch_events() {
 __global__ __launch_bounds__(256) void k_minmax(const double* __restrict__ x, uint64_t n, uint64_t ntiles,
                                                 uint64_t tpw, int32_t pexp, uint32_t dlen,
                                                 int64_t* __restrict__ partial, int64_t* __restrict__ set,
-                                                int64_t* __restrict__ next) {
+                                                int64_t* __restrict__ next, Publish pub) {
   const uint32_t lane = __lane_id();
   const uint32_t wave = wave_in_wg();
   const uint64_t t0 = (uint64_t)blockIdx.x * tpw;
@@ -68,6 +96,31 @@ __global__ __launch_bounds__(256) void k_minmax(const double* __restrict__ x, ui
   __shared__ int64_t smn[4], smx[4];
   if (lane == 0) { smn[wave] = mn; smx[wave] = mx; }
   __syncthreads();
+  if (pub.mbox) {   // set is handed over here and left empty
+    if (wave != 0) return;
+    int64_t a = min(min(smn[0], smn[1]), min(smn[2], smn[3]));
+    int64_t b = max(max(smx[0], smx[1]), max(smx[2], smx[3]));
+    if (lane == 0) {
+      partial[blockIdx.x] = a;   // kept for the prefix-min pass
+      partial[gridDim.x + blockIdx.x] = b;
+    }
+    if (gridDim.x > 1) {
+      if (lane == 0) {
+        const uint32_t slot = blockIdx.x % kMinMaxSlots;
+        if (a != INT64_MAX) (void)atomicMin((long long*)&set[slot], (long long)a);
+        if (b != INT64_MIN) (void)atomicMax((long long*)&set[kMinMaxSlots + slot], (long long)b);
+      }
+      if (!last_workgroup((unsigned long long*)&set[kMinMaxTicket])) return;
+      a = wave_min_i64(slot_load(&set[lane]));
+      b = wave_max_i64(slot_load(&set[kMinMaxSlots + lane]));
+      set[lane] = INT64_MAX;
+      set[kMinMaxSlots + lane] = INT64_MIN;
+      if (lane == 0) set[kMinMaxTicket] = 0;
+    }
+    const int64_t f0 = fetch_fixed_aligned_bits(__double_as_longlong(x[0]), pexp, dlen);
+    publish_words(pub, (uint64_t)(lane == 0 ? a : lane == 1 ? b : f0), 3);
+    return;
+  }
   if (threadIdx.x == 0) {
     const int64_t a = min(min(smn[0], smn[1]), min(smn[2], smn[3]));
     const int64_t b = max(max(smx[0], smx[1]), max(smx[2], smx[3]));
@@ -437,7 +490,7 @@ __global__ void k_touch_bytes(const uint4* __restrict__ in, uint64_t n16, uint32
 
 template <int P, int R, int U>
 __global__ __launch_bounds__(256) void k_sum(ChunkView cv, unsigned long long* __restrict__ rows,
-                                             unsigned long long* __restrict__ next) {
+                                             unsigned long long* __restrict__ next, Publish pub) {
   const uint32_t lane = __lane_id();
   const uint64_t wave = wave_global();
   const uint64_t nwaves = waves_in_grid();
@@ -501,6 +554,29 @@ __global__ __launch_bounds__(256) void k_sum(ChunkView cv, unsigned long long* _
   t = wave_sum_u64(t);
   if (lane == 0) wrow[wslot][P] = t;
   __syncthreads();
+  if (pub.mbox) {   // the slot set `rows` is handed over here and left zero
+    if (wslot != 0) return;
+    uint64_t v = 0;
+    if (lane <= (uint32_t)P)
+      for (uint32_t k = 0; k < (blockDim.x >> 6); ++k) v += wrow[k][lane];
+    if (gridDim.x > 1) {
+      if (lane <= (uint32_t)P && v)
+        (void)atomicAdd(&rows[lane * kSumSlots + blockIdx.x % kSumSlots], (unsigned long long)v);
+      if (!last_workgroup(&rows[kSumTicket])) return;
+      uint64_t part[P + 1];   // all loads in flight together
+#pragma unroll
+      for (uint32_t k = 0; k <= (uint32_t)P; ++k) part[k] = slot_load(&rows[k * kSumSlots + lane]);
+#pragma unroll
+      for (uint32_t k = 0; k <= (uint32_t)P; ++k) {
+        const uint64_t s = wave_sum_u64(part[k]);
+        if (lane == k) v = s;
+        rows[k * kSumSlots + lane] = 0ull;
+      }
+      if (lane == 0) rows[kSumTicket] = 0ull;
+    }
+    publish_words(pub, v, P + 1);
+    return;
+  }
   if (threadIdx.x <= (uint32_t)P) {
     uint64_t v = 0;
     for (uint32_t k = 0; k < (blockDim.x >> 6); ++k) v += wrow[k][threadIdx.x];
@@ -701,6 +777,34 @@ __global__ __launch_bounds__(256) void k_max_refine(ChunkView cv, const uint8_t*
     const unsigned long long b = max(max(wbest[0], wbest[1]), max(wbest[2], wbest[3]));
     if (b && b - 1 > __hip_atomic_load(best_out, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) atomicMax(best_out, b - 1);
   }
+}
+
+// Small columns (at most kMaxDirectTiles tiles): a wave rebuilds its tiles'
+// offsets at once, without a pass over the top bytes first, and the last
+// workgroup publishes: bound by the launch, so one instead of three (a call on
+// 4097 rows 15.2 -> 11.3 us, on 1M 15.5 -> 13.9; above, the top bytes alone are
+// quicker read).
+__global__ __launch_bounds__(256) void k_max_direct(ChunkView cv, unsigned long long* __restrict__ set, Publish pub) {
+  const uint32_t lane = __lane_id(), wave = wave_in_wg();
+  uint64_t m = 0;
+  for (uint64_t c = wave_global(); c < cv.ntiles; c += waves_in_grid()) {
+    const uint64_t t = lane_max_offset(cv, c, lane);
+    m = t > m ? t : m;
+  }
+  __shared__ unsigned long long wbest[4];
+  m = wave_max_u64(m);
+  if (lane == 0) wbest[wave] = m;
+  __syncthreads();
+  if (wave != 0) return;
+  unsigned long long b = max(max(wbest[0], wbest[1]), max(wbest[2], wbest[3]));
+  if (gridDim.x > 1) {
+    if (lane == 0 && b) (void)atomicMax(&set[blockIdx.x % kSumSlots], b);
+    if (!last_workgroup(&set[kSumTicket])) return;
+    b = wave_max_u64(slot_load(&set[lane]));
+    set[lane] = 0ull;
+    if (lane == 0) set[kSumTicket] = 0ull;
+  }
+  publish_words(pub, b, 1);
 }
 
 // One pass (a tuner choice; the two-pass form below is the default): every
@@ -1027,6 +1131,8 @@ static inline uint32_t grid_for(uint64_t units, uint32_t waves_per_wg, uint32_t 
 }
 
 uint32_t minmax_grid(uint64_t ntiles) {
+  // few tiles: one a wave, so that the launch hands its result over itself
+  if (ntiles <= 4 * kFusedWgs) return (uint32_t)std::max<uint64_t>(1, (ntiles + 3) / 4);
   // 1024 workgroups (16 waves per CU) measured faster than the ~1800 that fit
   return (uint32_t)std::max<uint64_t>(1, std::min<uint64_t>({ntiles, 1024, resident_wgs(k_minmax, 256)}));
 }
@@ -1037,7 +1143,7 @@ hipError_t launch_minmax(const double* x, uint64_t n, int32_t pexp, uint32_t dle
   const uint64_t tpw = (ntiles + nwg - 1) / nwg;
   if (!prefix) {
     launch_k(k_minmax, dim3(nwg), dim3(256), 0, s, x, n, ntiles, tpw, pexp, dlen, partial, (int64_t*)nullptr,
-             (int64_t*)nullptr);
+             (int64_t*)nullptr, Publish{});
     launch_k(k_minmax_final, dim3(1), dim3(256), 0, s, x, n, pexp, dlen, (const int64_t*)partial, nwg,
                        out);
   } else {
@@ -1049,11 +1155,15 @@ hipError_t launch_minmax(const double* x, uint64_t n, int32_t pexp, uint32_t dle
 }
 
 hipError_t launch_minmax_slots(const double* x, uint64_t n, int32_t pexp, uint32_t dlen, int64_t* partial,
-                               int64_t* set, int64_t* next, uint32_t nwg, hipStream_t s) {
+                               int64_t* set, int64_t* next, uint32_t nwg, hipStream_t s, const Publish* pub,
+                               bool* published) {
   if (!set || !next || n == 0) return hipErrorInvalidValue;
   const uint64_t ntiles = (n + kTileRows - 1) / kTileRows;
   const uint64_t tpw = (ntiles + nwg - 1) / nwg;
-  launch_k(k_minmax, dim3(nwg), dim3(256), 0, s, x, n, ntiles, tpw, pexp, dlen, partial, set, next);
+  const bool fused = pub && nwg <= kFusedWgs;
+  if (published) *published = fused;
+  launch_k(k_minmax, dim3(nwg), dim3(256), 0, s, x, n, ntiles, tpw, pexp, dlen, partial, set, next,
+           fused ? *pub : Publish{});
   return hipGetLastError();
 }
 
@@ -1078,10 +1188,7 @@ __global__ __launch_bounds__(64) void k_publish(const uint64_t* __restrict__ src
   } else if (lane < nk) {
     mine = src[lane];
   }
-  if (lane < nw) pub.mbox[1 + lane] = mine;
-  __threadfence_system();
-  __syncthreads();
-  if (lane == 0) __hip_atomic_store(pub.mbox, pub.seq, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+  publish_words(pub, mine, nw);
 }
 
 hipError_t launch_publish(const void* src, uint32_t mode, uint32_t nk, const Publish& pub, hipStream_t s) {
@@ -1221,28 +1328,30 @@ hipError_t launch_touch_bytes(const void* in, uint64_t bytes, uint32_t* sink, hi
 // k_sum_final into sums; else one launch adding into the slot set `sums`.
 template <int P, int R, int U>
 static void launch_sum_pru(const ChunkView& cv, unsigned long long* sums, unsigned long long* next, hipStream_t s,
-                           const LaunchShape& ls) {
+                           const LaunchShape& ls, const Publish* pub, bool* published) {
   const uint32_t block = 64 * ls.waves_per_wg;
   const uint32_t wg = std::min<uint32_t>(
       grid_for((cv.ntiles + U - 1) / U, ls.waves_per_wg, cap_of(ls, resident_wgs(k_sum<P, R, U>, block))),
       kMaxSumRows);
   if (next) {
-    launch_k((k_sum<P, R, U>), dim3(wg), dim3(block), 0, s, cv, sums, next);
+    const bool fused = pub && wg <= kFusedWgs;
+    if (published) *published = fused;
+    launch_k((k_sum<P, R, U>), dim3(wg), dim3(block), 0, s, cv, sums, next, fused ? *pub : Publish{});
     return;
   }
   unsigned long long* rows = sums + (kMaxPlanes + 1);
-  launch_k((k_sum<P, R, U>), dim3(wg), dim3(block), 0, s, cv, rows, (unsigned long long*)nullptr);
+  launch_k((k_sum<P, R, U>), dim3(wg), dim3(block), 0, s, cv, rows, (unsigned long long*)nullptr, Publish{});
   launch_k((k_sum_final<P + 1>), dim3(1), dim3(256), 0, s, (const unsigned long long*)rows, wg, sums);
 }
 
 template <int P, int R>
 static void launch_sum_pr(const ChunkView& cv, unsigned long long* sums, unsigned long long* next, hipStream_t s,
-                          const LaunchShape& ls) {
+                          const LaunchShape& ls, const Publish* pub, bool* published) {
   switch (ls.tiles_per_wave) {
-    case 1: launch_sum_pru<P, R, 1>(cv, sums, next, s, ls); break;
-    case 2: launch_sum_pru<P, R, 2>(cv, sums, next, s, ls); break;
-    case 4: launch_sum_pru<P, R, 4>(cv, sums, next, s, ls); break;
-    default: launch_sum_pru<P, R, (P + R) <= 3 ? 4 : 2>(cv, sums, next, s, ls); break;
+    case 1: launch_sum_pru<P, R, 1>(cv, sums, next, s, ls, pub, published); break;
+    case 2: launch_sum_pru<P, R, 2>(cv, sums, next, s, ls, pub, published); break;
+    case 4: launch_sum_pru<P, R, 4>(cv, sums, next, s, ls, pub, published); break;
+    default: launch_sum_pru<P, R, (P + R) <= 3 ? 4 : 2>(cv, sums, next, s, ls, pub, published); break;
   }
 }
 
@@ -1253,44 +1362,44 @@ uint64_t sum_scratch_bytes(const LaunchShape& ls) {
 
 template <int P>
 static hipError_t launch_sum_p(const ChunkView& cv, unsigned long long* sums, unsigned long long* next, hipStream_t s,
-                               const LaunchShape& ls) {
+                               const LaunchShape& ls, const Publish* pub, bool* published) {
   switch (cv.r) {
-    case 0: launch_sum_pr<P, 0>(cv, sums, next, s, ls); break;
-    case 1: launch_sum_pr<P, 1>(cv, sums, next, s, ls); break;
-    case 2: launch_sum_pr<P, 2>(cv, sums, next, s, ls); break;
-    case 3: launch_sum_pr<P, 3>(cv, sums, next, s, ls); break;
-    case 4: launch_sum_pr<P, 4>(cv, sums, next, s, ls); break;
-    case 5: launch_sum_pr<P, 5>(cv, sums, next, s, ls); break;
-    case 6: launch_sum_pr<P, 6>(cv, sums, next, s, ls); break;
-    case 7: launch_sum_pr<P, 7>(cv, sums, next, s, ls); break;
+    case 0: launch_sum_pr<P, 0>(cv, sums, next, s, ls, pub, published); break;
+    case 1: launch_sum_pr<P, 1>(cv, sums, next, s, ls, pub, published); break;
+    case 2: launch_sum_pr<P, 2>(cv, sums, next, s, ls, pub, published); break;
+    case 3: launch_sum_pr<P, 3>(cv, sums, next, s, ls, pub, published); break;
+    case 4: launch_sum_pr<P, 4>(cv, sums, next, s, ls, pub, published); break;
+    case 5: launch_sum_pr<P, 5>(cv, sums, next, s, ls, pub, published); break;
+    case 6: launch_sum_pr<P, 6>(cv, sums, next, s, ls, pub, published); break;
+    case 7: launch_sum_pr<P, 7>(cv, sums, next, s, ls, pub, published); break;
     default: return hipErrorInvalidValue;
   }
   return hipGetLastError();
 }
 
 static hipError_t launch_sum_any(const ChunkView& cv, unsigned long long* sums, unsigned long long* next,
-                                 hipStream_t s, const LaunchShape& ls) {
+                                 hipStream_t s, const LaunchShape& ls, const Publish* pub, bool* published) {
   switch (cv.P) {
-    case 0: return launch_sum_p<0>(cv, sums, next, s, ls);
-    case 1: return launch_sum_p<1>(cv, sums, next, s, ls);
-    case 2: return launch_sum_p<2>(cv, sums, next, s, ls);
-    case 3: return launch_sum_p<3>(cv, sums, next, s, ls);
-    case 4: return launch_sum_p<4>(cv, sums, next, s, ls);
-    case 5: return launch_sum_p<5>(cv, sums, next, s, ls);
-    case 6: return launch_sum_p<6>(cv, sums, next, s, ls);
-    case 7: return launch_sum_p<7>(cv, sums, next, s, ls);
+    case 0: return launch_sum_p<0>(cv, sums, next, s, ls, pub, published);
+    case 1: return launch_sum_p<1>(cv, sums, next, s, ls, pub, published);
+    case 2: return launch_sum_p<2>(cv, sums, next, s, ls, pub, published);
+    case 3: return launch_sum_p<3>(cv, sums, next, s, ls, pub, published);
+    case 4: return launch_sum_p<4>(cv, sums, next, s, ls, pub, published);
+    case 5: return launch_sum_p<5>(cv, sums, next, s, ls, pub, published);
+    case 6: return launch_sum_p<6>(cv, sums, next, s, ls, pub, published);
+    case 7: return launch_sum_p<7>(cv, sums, next, s, ls, pub, published);
     default: return hipErrorInvalidValue;
   }
 }
 
 hipError_t launch_sum(const ChunkView& cv, unsigned long long* sums, hipStream_t s, const LaunchShape& ls) {
-  return launch_sum_any(cv, sums, nullptr, s, ls);
+  return launch_sum_any(cv, sums, nullptr, s, ls, nullptr, nullptr);
 }
 
 hipError_t launch_sum_slots(const ChunkView& cv, unsigned long long* set, unsigned long long* next, hipStream_t s,
-                            const LaunchShape& ls) {
+                            const LaunchShape& ls, const Publish* pub, bool* published) {
   if (!set || !next) return hipErrorInvalidValue;
-  return launch_sum_any(cv, set, next, s, ls);
+  return launch_sum_any(cv, set, next, s, ls, pub, published);
 }
 
 uint64_t max_scratch_bytes(uint64_t ntiles) { return ((ntiles + 255) / 256) * 256; }
@@ -1342,6 +1451,12 @@ hipError_t launch_max(const ChunkView& cv, unsigned long long* best, uint8_t* sc
   const uint32_t wg2 = grid_for((cv.ntiles + T - 1) / T, 4, fit);
   launch_k(k_max_refine, dim3(wg2), dim3(256), 0, s, cv, (const uint8_t*)scratch, (const unsigned int*)slots, tag, T,
            best);
+  return hipGetLastError();
+}
+
+hipError_t launch_max_direct(const ChunkView& cv, unsigned long long* set, const Publish& pub, hipStream_t s) {
+  if (!set || !pub.mbox || cv.ntiles == 0 || cv.ntiles > kMaxDirectTiles) return hipErrorInvalidValue;
+  launch_k(k_max_direct, dim3(grid_for(cv.ntiles, 4, kFusedWgs)), dim3(256), 0, s, cv, set, pub);
   return hipGetLastError();
 }
 

@@ -117,6 +117,7 @@ struct Ctx {
   // queues the hand-over of a reduction's result (launch_publish into the
   // mailbox made with the context); published() waits until it has arrived
   // (or the stream failed or ended without it) and copies its nw result words
+  Publish next_publish();   // for a launch that publishes by itself
   int publish(const void* src, uint32_t mode, uint32_t nk, Publish* pub);
   int published(const Publish& pub, uint64_t* words, uint32_t nw);
   void prof_begin(const char* name, hipEvent_t* ev, bool kernels);

@@ -139,3 +139,25 @@ def test_csv_many_blocks(ctx):
     text[99::100, 8] = ord("\n")
     assert np.array_equal(ctx.csv_parse(text.tobytes()), k.astype(np.float64))
     assert np.array_equal(ctx.csv_parse(text.tobytes(), skip_val=3), k.reshape(-1, 100)[:, 3:].ravel().astype(np.float64))
+
+
+# sums, maxima and encodes whose result the last workgroup hands over (one workgroup, a few, 256), and the ones around
+# that take a second launch; interleaved, so that every call finds the slots as the one before left them
+@pytest.mark.parametrize("decimals", [1, 4, 8])
+def test_handover(ctx, decimals):
+    cols = []
+    for i, rows in enumerate((3, TILE, 4 * TILE + 1, 1000 * TILE, 1024 * TILE, 1024 * TILE + 1, 4096 * TILE, 4100 * TILE)):
+        x = datagen.random_walk(rows, decimals, 31 + i)
+        f = fixed(x, ctx_dlen := {1: 5, 4: 15, 8: 28}[decimals])
+        cols.append((x, f, ctx_dlen))
+    for rep in range(3):
+        for x, f, dlen in cols[::-1] if rep == 1 else cols:
+            ch = ctx.encode(x, 10 ** decimals)
+            info = ch.info()
+            assert info.base == f.min() and info.dlen == dlen
+            _, exact, _ = ch.sum()
+            assert exact == float(f.sum()) / 2.0 ** dlen
+            if f[0] < f.max():   # row 0 as the unique maximum is the header's own rule
+                assert ch.max()[0] == f.max() / 2.0 ** dlen
+            assert ch.sum()[1] == exact
+            ch.free()
