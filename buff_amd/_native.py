@@ -6,7 +6,9 @@ fallback; loading fails loudly when the library is missing.
 """
 import collections.abc
 import ctypes
+import operator
 import os
+import threading
 
 import numpy as np
 
@@ -498,6 +500,46 @@ class QueryResults(collections.abc.Sequence):
         return self._res[i]
 
 
+class _BatchChunks(collections.abc.Sequence):
+    """The chunks of a batch, each made when it is first asked for (a batch of hundreds is often only queried)."""
+
+    def __init__(self, ctx, batch, n):
+        self._ctx = ctx
+        self._batch = batch
+        self._chunks = [None] * n
+        self._lock = threading.Lock()
+
+    def __len__(self):
+        return len(self._chunks)
+
+    def __getitem__(self, i):
+        if isinstance(i, slice):
+            return [self[k] for k in range(*i.indices(len(self._chunks)))]
+        i = operator.index(i)
+        if self._chunks[i] is None:
+            with self._lock:
+                if self._chunks[i] is None:
+                    h = ctypes.c_void_p()
+                    if self._batch is not None:
+                        check(lib().buff_batch_chunk(self._batch, i % len(self._chunks), ctypes.byref(h)))
+                    self._chunks[i] = Chunk(self._ctx, h.value, borrowed=True)
+        return self._chunks[i]
+
+    def __add__(self, other):
+        return list(self) + list(other)
+
+    def __radd__(self, other):
+        return list(other) + list(self)
+
+    def drop(self):
+        """The batch goes: its chunks have no handle any more."""
+        with self._lock:
+            self._batch = None
+            for c in self._chunks:
+                if c is not None:
+                    c.handle = None
+
+
 class Batch:
     """buff_batch*: chunks encoded together; queries over them run as one graph launch."""
 
@@ -506,11 +548,7 @@ class Batch:
         self.handle = handle
         n = ctypes.c_uint32()
         check(lib().buff_batch_size(handle, ctypes.byref(n)))
-        self.chunks = []
-        for i in range(n.value):
-            h = ctypes.c_void_p()
-            check(lib().buff_batch_chunk(handle, i, ctypes.byref(h)))
-            self.chunks.append(Chunk(ctx, h.value, borrowed=True))
+        self.chunks = _BatchChunks(ctx, handle, n.value)
 
     def query(self, qs):
         """Returns a list of QueryResult (see include/buffgpu.h)."""
@@ -549,8 +587,7 @@ class Batch:
 
     def free(self):
         if self.handle:
-            for c in self.chunks:
-                c.handle = None
+            self.chunks.drop()
             check(lib().buff_batch_free(self.handle))
             self.handle = None
 

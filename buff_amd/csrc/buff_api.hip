@@ -7,6 +7,7 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <array>
 #include <cstdarg>
 #include <cmath>
 #include <cstdio>
@@ -60,7 +61,7 @@ int precision_map(int p) {  // database/src/compress/mod.rs:29-46
   return (p >= 1 && p <= 15) ? tab[p] : -1;
 }
 
-int32_t precision_exp_of_prec(int prec) {  // prec_double.rs:28-33 of get_precision_bound(p), 273-281
+static int32_t bound_exponent(int prec) {
   std::string s = "0.";
   for (int i = 0; i < prec; ++i) s.push_back('0');
   s += "49";
@@ -68,6 +69,16 @@ int32_t precision_exp_of_prec(int prec) {  // prec_double.rs:28-33 of get_precis
   uint64_t u;
   memcpy(&u, &b, 8);
   return (int32_t)((u & 0x7FF0000000000000ull) >> 52) - 1023;
+}
+
+int32_t precision_exp_of_prec(int prec) {  // prec_double.rs:28-33 of get_precision_bound(p), 273-281
+  constexpr int kTab = 20;                 // every scale a u64 can hold
+  static const std::array<int32_t, kTab> tab = [] {
+    std::array<int32_t, kTab> t;
+    for (int p = 0; p < kTab; ++p) t[p] = bound_exponent(p);
+    return t;
+  }();
+  return prec >= 0 && prec < kTab ? tab[prec] : bound_exponent(prec);
 }
 
 double powi2(int32_t e) {  // 2.0f64.powi(e) as lowered by compiler-rt __powidf2
@@ -99,6 +110,7 @@ Ctx::~Ctx() {
   if (stream) {
     (void)hipStreamSynchronize(stream);
   }
+  if (spare_exec) spare_exec_free(spare_exec);
   for (auto& kv : free_blocks) (void)hipFree(kv.second);
   free_blocks.clear();
   for (auto& p : prof_pool) (void)hipEventDestroy(p);

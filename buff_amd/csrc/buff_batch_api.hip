@@ -343,6 +343,56 @@ void exec_free(QueryExec& ex) {
   ex.stream = nullptr;
 }
 
+// A freed batch's executor stays with its context (one at most, of bounded
+// staging and graphs): a program that encodes, queries and drops batch after
+// batch does not capture its graphs and pin its staging again each time. Its
+// device buffers go back to the context's cache except the one the graphs read
+// their addresses from; the next batch uploads its own addresses into that.
+constexpr uint32_t kSparePinQueries = 1u << 16;
+constexpr size_t kSpareGraphs = 32;
+
+void exec_park(QueryExec& ex) {
+  if (!ex.ctx) return;
+  Ctx* ctx = ex.ctx;
+  QueryExec* spare = nullptr;
+  if (ex.done && !ex.own_stream && !ex.aux && ex.pin_cap <= kSparePinQueries && ex.graphs.size() <= kSpareGraphs)
+    spare = new (std::nothrow) QueryExec();
+  if (!spare) {
+    exec_free(ex);
+    return;
+  }
+  (void)hipStreamSynchronize(ex.stream);
+  for (DevBuf* d : {&ex.hdr, &ex.q, &ex.items, &ex.acc, &ex.res, &ex.top, &ex.arena}) drop(ctx, *d);
+  *spare = std::move(ex);
+  ex = QueryExec{};
+  {
+    std::lock_guard<std::mutex> lk(ctx->mu);
+    if (!ctx->spare_exec) {
+      ctx->spare_exec = spare;
+      ctx->spare_exec_free = [](void* p) {
+        exec_free(*static_cast<QueryExec*>(p));
+        delete static_cast<QueryExec*>(p);
+      };
+      return;
+    }
+  }
+  exec_free(*spare);
+  delete spare;
+}
+
+int exec_take(QueryExec& ex, Ctx* ctx) {
+  QueryExec* spare;
+  {
+    std::lock_guard<std::mutex> lk(ctx->mu);
+    spare = static_cast<QueryExec*>(ctx->spare_exec);
+    ctx->spare_exec = nullptr;
+  }
+  if (!spare) return exec_init(ex, ctx, false);
+  ex = std::move(*spare);
+  delete spare;
+  return BUFF_OK;
+}
+
 int graph_for(QueryExec& ex, const BatchTuning& tu, uint32_t parts, hipGraphExec_t* out) {
   const uint64_t key = ((uint64_t)tu.grid << 32) | ((uint64_t)parts << 16) | tu.first_planes;
   auto it = ex.graphs.find(key);
@@ -691,7 +741,7 @@ int batch_query(Ctx* ctx, Batch* b, const buff_query* qs, uint32_t nq, buff_quer
                 const BatchTuning& tu, float* graph_ms) {
   if (!ctx || !b || (nq && (!qs || !results))) return fail(BUFF_E_INVALID, "null argument");
   if (b->ctx != ctx) return fail(BUFF_E_INVALID, "the batch belongs to another context");
-  if (!b->ex.ctx) BUFF_TRY(exec_init(b->ex, ctx, false));
+  if (!b->ex.ctx) BUFF_TRY(exec_take(b->ex, ctx));
   hipEvent_t ev0 = nullptr;
   if (graph_ms) {
     HIP_TRY(hipEventCreate(&ev0));
@@ -729,7 +779,7 @@ int batch_query(Ctx* ctx, Batch* b, const buff_query* qs, uint32_t nq, buff_quer
 void batch_free(Batch* b) {
   Ctx* ctx = b->ctx;
   (void)hipStreamSynchronize(ctx->stream);
-  exec_free(b->ex);
+  exec_park(b->ex);
   for (Chunk* ch : b->chunks) delete ch;
   drop(ctx, b->pool);
   drop(ctx, b->views);

@@ -88,6 +88,11 @@ struct Ctx {
   std::vector<ProfRec> prof_pending;
   std::map<std::string, std::pair<uint64_t, double>> prof_stats;
 
+  // the executor (captured graphs, pinned staging) of the last freed batch, for
+  // the next batch's first query; ended with the context (mu)
+  void* spare_exec = nullptr;
+  void (*spare_exec_free)(void*) = nullptr;
+
   std::map<uint64_t, LaunchShape> tuned;
   // batched queries: grid, tiles per work item, planes of the first filter pass.
   // The grid is twice what is resident: the workgroups beyond it start as

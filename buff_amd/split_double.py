@@ -32,12 +32,19 @@ class SplitBDDoubleCompress:
 
     def _encode(self, fn, data):
         x = np.ascontiguousarray(data, dtype=np.float64)
-        L = N.lib()
         n = ctypes.c_uint64()
-        N.check(getattr(L, fn)(ctypes.byref(self._sd), N.ptr(x, ctypes.c_double), len(x), None, 0, ctypes.byref(n)))
-        out = np.zeros(n.value, dtype=np.uint8)
-        N.check(getattr(L, fn)(ctypes.byref(self._sd), N.ptr(x, ctypes.c_double), len(x), N.ptr(out, ctypes.c_uint8),
-                               len(out), ctypes.byref(n)))
+        # room for the 64 bits a row that a byte_fixed stream stays below, cut to the stream's size afterwards: asking
+        # for the size first would upload and encode the column twice. A sparse layout's stream can be longer; the
+        # call then names its size.
+        out = np.empty(8 * len(x) + 64, dtype=np.uint8)
+        for last in (False, True):
+            rc = getattr(N.lib(), fn)(ctypes.byref(self._sd), N.ptr(x, ctypes.c_double), len(x),
+                                      N.ptr(out, ctypes.c_uint8), len(out), ctypes.byref(n))
+            if rc != N.BUFF_E_SMALL_BUFFER or last:
+                break
+            out = np.empty(n.value, dtype=np.uint8)
+        N.check(rc)
+        out.resize(n.value, refcheck=False)
         return out
 
     def byte_fixed_encode(self, data):  # split_double.rs:298
@@ -49,7 +56,7 @@ class SplitBDDoubleCompress:
     def _decode(self, fn, b, *extra):
         b = _u8(b)
         n = _stream_n(b)
-        out = np.zeros(max(n, 1), dtype=np.float64)
+        out = np.empty(max(n, 1), dtype=np.float64)   # every value is written
         N.check(getattr(N.lib(), fn)(ctypes.byref(self._sd), N.ptr(b, ctypes.c_uint8), len(b), *extra,
                                      N.ptr(out, ctypes.c_double), len(out)))
         return out[:n]
@@ -65,7 +72,7 @@ class SplitBDDoubleCompress:
 
     def _residue_decode(self, fn, b, *extra):
         b = _u8(b)
-        out = np.zeros(max(_stream_n(b), 1), dtype=np.float64)
+        out = np.empty(max(_stream_n(b), 1), dtype=np.float64)   # the first `got` values are written
         got = ctypes.c_uint64()
         N.check(getattr(N.lib(), fn)(ctypes.byref(self._sd), N.ptr(b, ctypes.c_uint8), len(b), *extra,
                                      N.ptr(out, ctypes.c_double), len(out), ctypes.byref(got)))
@@ -134,7 +141,7 @@ class SplitBDDoubleCompress:
     def buff_decode_majority(self, b):  # buff_simd.rs:633 (empty when the stream ends in sparse columns)
         b = _u8(b)
         n = _stream_n(b)
-        out = np.zeros(max(n, 1), dtype=np.float64)
+        out = np.empty(max(n, 1), dtype=np.float64)   # the first `got` values are written
         got = ctypes.c_uint64()
         N.check(N.lib().buff_sd_buff_decode_majority(ctypes.byref(self._sd), N.ptr(b, ctypes.c_uint8), len(b),
                                                      N.ptr(out, ctypes.c_double), len(out), ctypes.byref(got)))

@@ -5,7 +5,9 @@ import numpy as np
 import pytest
 
 import buff_amd
+from buff_amd import _native as N
 from buff_amd import datagen
+from buff_amd.split_double import SplitBDDoubleCompress
 from oracle import refcpu, refcsv
 
 pytestmark = pytest.mark.gpu
@@ -161,3 +163,65 @@ def test_handover(ctx, decimals):
                 assert ch.max()[0] == f.max() / 2.0 ** dlen
             assert ch.sum()[1] == exact
             ch.free()
+
+
+# batch after batch on one context (the second and third take over the first's executor), two alive at once, larger
+# and smaller query lists: every answer from its own batch's chunks; chunk handles made on demand
+def test_batch_after_batch(ctx):
+    def encode(seed, lens):
+        cols = [datagen.uniform(n, -1000, 1000, 3, seed + i) for i, n in enumerate(lens)]
+        off = np.concatenate([[0], np.cumsum(lens)]).astype(np.uint64)
+        xd = ctx.alloc(8 * int(off[-1]))
+        xd.upload(np.concatenate(cols))
+        b = ctx.batch_encode_device(xd.ptr, off, np.full(len(lens), 1000, dtype=np.uint64))
+        xd.free()
+        return b, cols
+
+    def check(b, cols, reps):
+        qs = [(N.BUFF_Q_SUM, k % len(cols), 0.0, -1, 0) for k in range(len(cols) * reps)]
+        qs += [(N.BUFF_Q_GT, k, float(c[0]), -1, N.BUFF_SEMANTIC) for k, c in enumerate(cols)]
+        res = b.query(qs)
+        for k, r in enumerate(res):
+            f = fixed(cols[k % len(cols)], 11)
+            if k < len(cols) * reps:
+                assert r.exact == float(f.sum()) / 2.0 ** 11
+            else:
+                assert r.count == (f > f[0]).sum()
+                assert np.array_equal(bits(b.bitmap(r, len(f)), len(f)), f > f[0])
+
+    first, a = encode(1, [1500, 30, 40_000])
+    check(first, a, 1)
+    last = first.chunks[-1]
+    assert len(first.chunks) == 3 and last is first.chunks[2] and last.info().n == 40_000
+    assert [c.info().n for c in first.chunks] == [1500, 30, 40_000]
+    with pytest.raises(IndexError):
+        first.chunks[3]
+    first.free()
+    assert last.handle is None
+    second, b = encode(50, [70_001, 20])
+    third, c = encode(90, [1024] * 9)
+    for reps in (1, 300, 1):
+        check(second, b, reps)
+        check(third, c, reps)
+    third.free()
+    second.free()
+    fourth, d = encode(130, [50, 2_000_000])
+    check(fourth, d, 20)
+    fourth.free()
+
+
+# the host codec's streams, whatever their length against the room their first call gives
+@pytest.mark.parametrize("rows", [2, 3, 63, 64, 65, 1024, 5000])
+@pytest.mark.parametrize("decimals", [1, 3, 12])
+def test_codec_sizes(ctx, rows, decimals):
+    scale = 10 ** decimals
+    comp = SplitBDDoubleCompress(rows, rows, scale)
+    x = np.append(datagen.uniform(rows - 1, -1000, 1000, min(decimals, 4), rows), 1000.25)
+    for name, flags in (("byte_fixed_encode", 0), ("byte_residue_encode", buff_amd.BUFF_RESIDUE),
+                        ("buff_encode_majority", buff_amd.BUFF_MAJORITY)):
+        if flags == buff_amd.BUFF_MAJORITY and rows < 2000:   # its sample
+            continue
+        ch = ctx.encode(x, scale, flags=flags)
+        got = getattr(comp, name)(x)
+        assert got.flags.owndata and np.array_equal(got, ch.serialize())
+        ch.free()
