@@ -433,8 +433,8 @@ int d2h_small(Ctx* ctx, void* dst, const void* src, uint64_t bytes) {
 
 // The running min and `else if` max of split_double.rs:321-330 over n rows of
 // device memory (n == 0: INT64_MAX / INT64_MIN, as the reference's initial values).
-int quirk_minmax(Ctx* ctx, const double* x, uint64_t n, int32_t pexp, uint32_t dlen, int64_t* mn_out,
-                 int64_t* mx_out) {
+static int quirk_minmax(Ctx* ctx, const double* x, uint64_t n, int32_t pexp, uint32_t dlen, int64_t* mn_out,
+                        int64_t* mx_out) {
   int64_t mn = INT64_MAX, mx = INT64_MIN;
   if (n > 0) {
     MinMaxOut mm;

@@ -36,16 +36,21 @@ struct BItem {
 static_assert(sizeof(BItem) == 24 && offsetof(BItem, chunk) == 4 && offsetof(BItem, c0) == 8, "BItem layout");
 
 // Per-chunk min/max of the `else if` pass (split_double.rs:321-330): min over all
-// rows, max over rows >= 1, and the fixed value of row 0.
+// rows, max over rows >= 1, the fixed value of row 0 and, when row 0 alone holds
+// the maximum, the max over the rows not below every row before them.
 struct BMinMax {
   int64_t min_all;
   int64_t max_rest;
   int64_t first;
-  int64_t pad;
+  int64_t qmax;
 };
 
+// Tiles of an encode item at most.
+constexpr uint32_t kEncodeItemTiles = 16;
+
+// list: 1 + nitems words of scratch.
 hipError_t launch_batch_minmax(const BEncChunk* chunks, uint32_t nchunks, const BItem* items, uint32_t nitems,
-                               int64_t* item_part, BMinMax* out, uint32_t grid, hipStream_t s);
+                               int64_t* item_part, BMinMax* out, uint32_t* list, uint32_t grid, hipStream_t s);
 hipError_t launch_batch_encode(const BEncChunk* chunks, const BItem* items, uint32_t nitems, uint32_t grid,
                                hipStream_t s);
 

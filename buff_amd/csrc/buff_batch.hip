@@ -15,8 +15,10 @@ namespace buffgpu {
 // than the chunk's row 0 (split_double.rs:321-330 keeps row 0 out of the max).
 
 __global__ __launch_bounds__(256) void k_bminmax(const BEncChunk* __restrict__ chunks, const BItem* __restrict__ items,
-                                                 uint32_t nitems, int64_t* __restrict__ part) {
+                                                 uint32_t nitems, int64_t* __restrict__ part,
+                                                 uint32_t* __restrict__ list) {
   __shared__ int64_t smn[4], smx[4];
+  if (blockIdx.x == 0 && threadIdx.x == 0) *list = 0;   // for k_bminmax_final
   const uint32_t lane = __lane_id(), wave = wave_in_wg();
   for (uint32_t i = blockIdx.x; i < nitems; i += gridDim.x) {
     const BItem it = items[i];
@@ -54,7 +56,8 @@ __global__ __launch_bounds__(256) void k_bminmax(const BEncChunk* __restrict__ c
 
 // One wave per chunk folds its items.
 __global__ __launch_bounds__(256) void k_bminmax_final(const BEncChunk* __restrict__ chunks, uint32_t nchunks,
-                                                       const int64_t* __restrict__ part, BMinMax* __restrict__ out) {
+                                                       const int64_t* __restrict__ part, BMinMax* __restrict__ out,
+                                                       uint32_t* __restrict__ list) {
   const uint32_t lane = __lane_id();
   const uint64_t wave = wave_global();
   const uint64_t nwaves = waves_in_grid();
@@ -67,13 +70,93 @@ __global__ __launch_bounds__(256) void k_bminmax_final(const BEncChunk* __restri
     }
     mn = wave_min_i64(mn);
     mx = wave_max_i64(mx);
+    const int64_t first = ck.view.n ? fetch_fixed_aligned_bits(__double_as_longlong(ck.x[0]), ck.pexp, ck.view.dlen) : 0;
+    if (ck.view.n > 1 && mx < first) {
+      uint32_t at = 0;
+      if (lane == 0) at = atomicAdd(list, ck.nitems);
+      at = __shfl(at, 0, 64);
+      for (uint32_t i = lane; i < ck.nitems; i += 64) list[1 + at + i] = ck.item0 + i;
+    }
     if (lane == 0) {
       BMinMax r;
       r.min_all = mn;
       r.max_rest = mx;
-      r.first = ck.view.n ? fetch_fixed_aligned_bits(__double_as_longlong(ck.x[0]), ck.pexp, ck.view.dlen) : 0;
-      r.pad = 0;
+      r.first = first;
+      r.qmax = INT64_MIN;
       out[k] = r;
+    }
+  }
+}
+
+// The max of chunks whose row 0 alone holds the maximum: over the rows not below
+// every row before them (the `else if` of split_double.rs:321-330), one
+// workgroup an item of such a chunk (k_bminmax_final lists them), one wave a
+// tile. The minimum before a wave's tile is the earlier items' and the earlier
+// waves', so all run at once; a group of 64 rows without a new minimum counts as
+// a whole, the others are scanned row by row. Launched always: without such
+// chunks it ends at once, and finding out on the host first would be a round
+// trip. 13 us for 512 walks of 1K to 1M rows, 3 of them such chunks; the
+// single-chunk replay from the host took 55 us of wall time for each of them, a
+// first version with four tiles a wave (read twice) 33 us in all.
+__global__ __launch_bounds__(64 * kEncodeItemTiles) void k_bminmax_prefix(const BEncChunk* __restrict__ chunks,
+                                                                          const BItem* __restrict__ items,
+                                                                          const int64_t* __restrict__ part,
+                                                                          const uint32_t* __restrict__ list,
+                                                                          BMinMax* __restrict__ out) {
+  __shared__ int64_t smn[kEncodeItemTiles], smx[kEncodeItemTiles];
+  const uint32_t lane = __lane_id(), wave = wave_in_wg();
+  const uint32_t total = *list;
+  for (uint32_t t = blockIdx.x; t < total; t += gridDim.x) {
+    const uint32_t i = list[1 + t];
+    const BItem it = items[i];
+    const BEncChunk& ck = chunks[it.owner];
+    const uint64_t n = ck.view.n, c = it.c0 + wave;
+    const bool mine = c < it.c1;
+    int64_t f[16], own = INT64_MAX;
+    if (mine) {
+      uint64_t v[16];
+      const bool full = tile_full(n, c);
+      load_tile_f64(ck.x, n, c, lane, full, v);
+#pragma unroll
+      for (uint32_t g = 0; g < 16; ++g) {
+        f[g] = full || c * kTileRows + 64 * g + lane < n ? fetch_fixed_aligned_bits(v[g], ck.pexp, ck.view.dlen)
+                                                         : INT64_MAX;
+        own = min(own, f[g]);
+      }
+    }
+    own = wave_min_i64(own);
+    if (lane == 0) smn[wave] = own;
+    int64_t carry = INT64_MAX;
+    for (uint32_t k = ck.item0 + lane; k < i; k += 64) carry = min(carry, part[2 * (uint64_t)k]);
+    carry = wave_min_i64(carry);
+    __syncthreads();
+    for (uint32_t w = 0; w < wave; ++w) carry = min(carry, smn[w]);
+    int64_t qmax = INT64_MIN;
+    if (mine) {
+#pragma unroll
+      for (uint32_t g = 0; g < 16; ++g) {
+        int64_t e = carry;
+        if (__any(f[g] < carry)) {
+          int64_t p = f[g];   // min over the lanes up to this one
+#pragma unroll
+          for (uint32_t o = 1; o < 64; o <<= 1) {
+            const int64_t u = (int64_t)__shfl_up((long long)p, o, 64);
+            if (lane >= o) p = min(p, u);
+          }
+          const int64_t u = (int64_t)__shfl_up((long long)p, 1, 64);
+          if (lane) e = min(carry, u);
+          carry = min(carry, (int64_t)__shfl((long long)p, 63, 64));
+        }
+        const bool valid = c * kTileRows + 64 * g + lane < n;
+        if (valid && f[g] >= e) qmax = max(qmax, f[g]);
+      }
+    }
+    qmax = wave_max_i64(qmax);
+    if (lane == 0) smx[wave] = qmax;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+      for (uint32_t w = 1; w < kEncodeItemTiles; ++w) qmax = max(qmax, smx[w]);
+      atomicMax((long long*)&out[it.owner].qmax, (long long)qmax);
     }
   }
 }
@@ -110,12 +193,16 @@ __global__ __launch_bounds__(256) void k_bencode(const BEncChunk* __restrict__ c
 }
 
 hipError_t launch_batch_minmax(const BEncChunk* chunks, uint32_t nchunks, const BItem* items, uint32_t nitems,
-                               int64_t* item_part, BMinMax* out, uint32_t grid, hipStream_t s) {
-  if (nitems) hipLaunchKernelGGL(k_bminmax, dim3(grid), dim3(256), 0, s, chunks, items, nitems, item_part);
+                               int64_t* item_part, BMinMax* out, uint32_t* list, uint32_t grid, hipStream_t s) {
+  if (nitems) hipLaunchKernelGGL(k_bminmax, dim3(grid), dim3(256), 0, s, chunks, items, nitems, item_part, list);
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) return e;
   hipLaunchKernelGGL(k_bminmax_final, dim3((nchunks + 3) / 4 ? (nchunks + 3) / 4 : 1), dim3(256), 0, s, chunks,
-                     nchunks, item_part, out);
+                     nchunks, item_part, out, list);
+  e = hipGetLastError();
+  if (e != hipSuccess || !nitems) return e;
+  hipLaunchKernelGGL(k_bminmax_prefix, dim3(nitems < 512 ? nitems : 512), dim3(64 * kEncodeItemTiles), 0, s, chunks,
+                     items, item_part, list, out);
   return hipGetLastError();
 }
 

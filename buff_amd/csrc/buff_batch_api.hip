@@ -106,8 +106,6 @@ struct Batch {
 
 namespace {
 
-constexpr uint64_t kEncodeItemTiles = 16;
-
 // ---------------------------------------------------------------------------
 // batch encode (byte_fixed_encode, split_double.rs:298-432, per chunk)
 
@@ -140,11 +138,12 @@ int batch_encode(Ctx* ctx, const double* x, const uint64_t* row_off, const uint6
     ck[i].nitems = (uint32_t)items.size() - ck[i].item0;
   }
   const uint32_t nitems = (uint32_t)items.size();
-  // scratch: [chunks | items | item partials | per-chunk min/max]
+  // scratch: [chunks | items | item partials | per-chunk min/max | items of chunks whose row 0 is the maximum]
   const uint64_t o_items = round_up(sizeof(BEncChunk) * std::max<uint32_t>(nchunks, 1), 256);
   const uint64_t o_part = o_items + round_up(sizeof(BItem) * std::max<uint32_t>(nitems, 1), 256);
   const uint64_t o_mm = o_part + round_up(16ull * std::max<uint32_t>(nitems, 1), 256);
-  const uint64_t total = o_mm + sizeof(BMinMax) * std::max<uint32_t>(nchunks, 1);
+  const uint64_t o_list = o_mm + round_up(sizeof(BMinMax) * std::max<uint32_t>(nchunks, 1), 256);
+  const uint64_t total = o_list + 4ull * (nitems + 1ull);
   BUFF_TRY(ctx->scratch(ctx->s_stream, total));
   uint8_t* sb = (uint8_t*)ctx->s_stream.ptr;
   BEncChunk* d_ck = (BEncChunk*)sb;
@@ -155,7 +154,7 @@ int batch_encode(Ctx* ctx, const double* x, const uint64_t* row_off, const uint6
     if (nitems) HIP_TRY(hipMemcpyAsync(d_items, items.data(), sizeof(BItem) * nitems, hipMemcpyHostToDevice, ctx->stream));
     {
       ProfScope ps(ctx, "k_batch_minmax", false);
-      HIP_TRY(launch_batch_minmax(d_ck, nchunks, d_items, nitems, (int64_t*)(sb + o_part), (BMinMax*)(sb + o_mm),
+      HIP_TRY(launch_batch_minmax(d_ck, nchunks, d_items, nitems, (int64_t*)(sb + o_part), (BMinMax*)(sb + o_mm), (uint32_t*)(sb + o_list),
                                   std::max<uint32_t>(1, std::min<uint32_t>(nitems, 4096)), ctx->stream));
     }
     HIP_TRY(hipMemcpyAsync(mm.data(), sb + o_mm, sizeof(BMinMax) * nchunks, hipMemcpyDeviceToHost, ctx->stream));
@@ -176,8 +175,7 @@ int batch_encode(Ctx* ctx, const double* x, const uint64_t* row_off, const uint6
       if (mm[i].max_rest >= mm[i].first) {
         mx = mm[i].max_rest;
       } else {
-        // row 0 holds the unique maximum: the single-chunk replay of the `else if`
-        BUFF_TRY(quirk_minmax(ctx, ck[i].x, n, ck[i].pexp, v.dlen, &mn, &mx));
+        mx = mm[i].first == INT64_MAX ? INT64_MAX : mm[i].qmax;
       }
     }
     const uint32_t F = width_of_delta((int64_t)((uint64_t)mx - (uint64_t)mn));

@@ -178,7 +178,6 @@ int d2h_small(Ctx* ctx, void* dst, const void* src, uint64_t bytes);
 int chunk_alloc(Ctx* ctx, Chunk* ch);
 void chunk_set_width(Chunk* ch, uint32_t F);
 int default_ctx(Ctx** out);
-int quirk_minmax(Ctx* ctx, const double* x, uint64_t n, int32_t pexp, uint32_t dlen, int64_t* mn, int64_t* mx);
 bool filter_plan(const Chunk* ch, int op, double pred, uint32_t flags, FilterTarget* tg, int* fill);
 double reference_sum_fold(const Chunk* ch, const uint64_t* ps);
 int mat_plan(const Chunk* ch, int32_t precision, uint32_t flags, MatParams* out);

@@ -225,3 +225,37 @@ def test_codec_sizes(ctx, rows, decimals):
         got = getattr(comp, name)(x)
         assert got.flags.owndata and np.array_equal(got, ch.serialize())
         ch.free()
+
+
+# chunks whose row 0 alone holds the maximum: new minima in the first rows only, all along (the fall of a walk) and at
+# the edges of groups, tiles, waves and 16-tile items; several such chunks among ordinary ones in one batch
+def test_batch_row0_max(ctx):
+    rng = np.random.default_rng(5)
+    cols = []
+    for n in (3, 64, 65, TILE, TILE + 1, 4 * TILE, 4 * TILE + 63, 15 * TILE + 1, 16 * TILE, 16 * TILE + 1, 64 * TILE + 9,
+              70 * TILE - 1):
+        fall = np.round(-np.arange(n) * 0.01 + rng.normal(0, 1, n), 2)
+        flat = np.round(rng.normal(0, 1, n), 2)
+        at = np.unique(np.clip([63, 64, TILE - 1, TILE, 4 * TILE - 1, 4 * TILE, 16 * TILE - 1, 16 * TILE], 1, n - 1))
+        edges = flat.copy()
+        edges[at] = -10.0 - np.arange(len(at))   # each a new minimum, the last but one row's maximum not
+        for x in (fall, flat, edges):
+            top = x.copy()
+            top[0] = x.max() + 2
+            cols += [top] if rng.random() < 0.9 else [top, x]
+    keep = []
+    for x in cols:
+        try:
+            keep.append((x, ctx.encode(x, 100)))
+        except N.RefPanic:   # no row counts into the maximum
+            pass
+    assert len(keep) > 30
+    off = np.concatenate([[0], np.cumsum([len(x) for x, _ in keep])]).astype(np.uint64)
+    xd = ctx.alloc(8 * int(off[-1]))
+    xd.upload(np.concatenate([x for x, _ in keep]))
+    b = ctx.batch_encode_device(xd.ptr, off, np.full(len(keep), 100, dtype=np.uint64))
+    xd.free()
+    for (x, ch), got in zip(keep, b.chunks):
+        assert np.array_equal(got.serialize(), ch.serialize()), len(x)
+        ch.free()
+    b.free()
