@@ -259,3 +259,51 @@ def test_batch_row0_max(ctx):
         assert np.array_equal(got.serialize(), ch.serialize()), len(x)
         ch.free()
     b.free()
+
+
+# the values of a condition's rows: offsets staged in 32 and in 64 bits (decimals), more tiles than waves, one range of
+# 64 tiles and many; dense, sparse and clustered conditions
+@pytest.mark.parametrize("decimals,rows", [(1, 1), (2, 1000), (2, 64 * TILE), (2, 64 * TILE + 1), (4, 8192 * TILE + 5),
+                                           (5, 5121 * TILE), (6, 6000 * TILE - 3), (12, 70 * TILE + 9)])
+def test_condition_values(ctx, decimals, rows):
+    rng = np.random.default_rng(rows)
+    x = rng.integers(-10 ** 5, 10 ** 5, rows) / 100.0
+    x[0] = x.min() - 1.5
+    if rows == 1:
+        with pytest.raises(N.RefPanic):
+            ctx.encode(x, 10 ** decimals)
+        return
+    ch = ctx.encode(x, 10 ** decimals)
+    dlen = ch.info().dlen
+    f = fixed(x, dlen)
+    for kind in ("dense", "sparse", "clustered", "none", "last"):
+        cond = np.zeros(rows, dtype=bool)
+        if kind == "dense":
+            cond[:] = rng.random(rows) < 0.9
+        elif kind == "sparse":
+            cond[rng.integers(0, rows, max(1, rows // 50))] = True
+        elif kind == "clustered":
+            cond[rows // 3: rows // 3 + rows // 7 + 1] = True
+        if kind != "none":
+            cond[-1] = True
+        words = np.packbits(cond, bitorder="little")
+        words = np.pad(words, (0, -len(words) % 8)).view(np.uint32)[: (rows + 31) // 32]
+        got = ch.materialize_cond(words, flags=buff_amd.BUFF_SEMANTIC)
+        assert np.array_equal(got, f[cond] / 2.0 ** dlen), kind
+    ch.free()
+
+
+# as many ranges as a wave adds up by itself, and one more
+@pytest.mark.parametrize("rows", [4096 * 64 * TILE, 4096 * 64 * TILE + 65])
+def test_condition_values_largest(ctx, rows):
+    x = (np.arange(rows, dtype=np.int32) * 7919 % 2001).astype(np.float64)
+    x[0] = -1.5
+    words = np.zeros((rows + 63) // 64, dtype=np.uint64)
+    at = np.random.default_rng(rows).integers(0, len(words) - 1, 100_000)
+    words[at] = 1 << 17   # a row of each of these words
+    words[-1] = 1
+    want = x[np.append(np.unique(at) * 64 + 17, (len(words) - 1) * 64)]
+    ch = ctx.encode(x, 10)
+    got = ch.materialize_cond(words.view(np.uint32)[: (rows + 31) // 32], flags=buff_amd.BUFF_SEMANTIC)
+    assert np.array_equal(got, want)
+    ch.free()
