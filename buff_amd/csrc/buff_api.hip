@@ -1479,7 +1479,7 @@ int tune_chunk(Ctx* ctx, const Chunk* ch, double pred, buff_tune_choice* out) {
     };
     buff_tune_choice ch_out{};
     ch_out.op = (uint32_t)op;
-    LaunchShape best{4, 0, 0};
+    LaunchShape best = default_shape(op, v.ntiles);
     float best_us = 0;
     rc = measure(best, &best_us);
     ch_out.default_us = best_us;
