@@ -217,7 +217,7 @@ __global__ __launch_bounds__(256) void k_major_filter(MajorPrefix<S> mv, MajorTa
   for (uint64_t grp = wave; grp < ngroups; grp += nwaves) {
     const uint64_t c0 = grp * U;
     uint32_t res[U];
-    major_filter_group<MODE, S, U, PF>(mv, tg, ru, c0, lane, dep, res);
+    major_filter_group<MODE, S, U, PF, MODE == 1 && !PF>(mv, tg, ru, c0, lane, dep, res);
 #pragma unroll
     for (int u = 0; u < U; ++u) {
       const uint64_t c = c0 + u;

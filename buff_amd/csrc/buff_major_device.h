@@ -216,7 +216,7 @@ __device__ __forceinline__ MajorRules<S> major_rules(const MV& mv, const MajorTa
 // for the candidates' lines in later dependent rounds.
 constexpr uint32_t kPfTail = 2;
 
-template <int MODE, int S, int U, bool PF = false, typename MV>
+template <int MODE, int S, int U, bool PF = false, bool RARE = false, typename MV>
 __device__ __forceinline__ void major_filter_group(const MV& mv, const MajorTarget& tg, const MajorRules<S>& ru,
                                                    uint64_t c0, uint32_t lane, unsigned long long* dep,
                                                    uint32_t (&res)[U]) {
@@ -246,6 +246,24 @@ __device__ __forceinline__ void major_filter_group(const MV& mv, const MajorTarg
       const bool has = lane < cnt[u][j];
       row0[u][j] = has ? mv.col[j].pos[p0[u][j] + lane] : 0u;
       byte0[u][j] = has ? mv.col[j].outl[p0[u][j] + lane] : 0u;
+    }
+  }
+  // RARE (equality where some sparse byte of the target is not the majority
+  // byte): if the first is not, only that column's outliers can match, and few
+  // tiles hold one that does: 40.4 us for such a value on 67,108,864 rows, 43.3
+  // with every tile deposited. A form of its own: the branch costs the others
+  // registers (equality with the majority value 42.6 -> 47.8).
+  if (RARE && S > 1 && ru.eqm[0] == 0) {
+    bool hit = false;
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      hit |= lane < cnt[u][0] && byte0[u][0] == tg.digit[0];
+      for (uint32_t k = lane + 64; k < cnt[u][0]; k += 64) hit |= mv.col[0].outl[p0[u][0] + k] == tg.digit[0];
+    }
+    if (__ballot(hit) == 0) {
+#pragma unroll
+      for (int u = 0; u < U; ++u) res[u] = 0;
+      return;
     }
   }
   uint32_t cand[U];
