@@ -92,10 +92,8 @@ __global__ __launch_bounds__(256) void k_bminmax_final(const BEncChunk* __restri
 // every row before them (the `else if` of split_double.rs:321-330), one
 // workgroup an item of such a chunk (k_bminmax_final lists them), one wave a
 // tile. The minimum before a wave's tile is the earlier items' and the earlier
-// waves', so all run at once; a group of 64 rows without a new minimum counts as
-// a whole, the others are scanned row by row. Launched always: without such
-// chunks it ends at once, and finding out on the host first would be a round
-// trip. 13 us for 512 walks of 1K to 1M rows, 3 of them such chunks; the
+// waves', so all run at once. Launched always: without such chunks it ends at
+// once, and finding out on the host first would be a round trip. 13 us for 512 walks of 1K to 1M rows, 3 of them such chunks; the
 // single-chunk replay from the host took 55 us of wall time for each of them, a
 // first version with four tiles a wave (read twice) 33 us in all.
 __global__ __launch_bounds__(64 * kEncodeItemTiles) void k_bminmax_prefix(const BEncChunk* __restrict__ chunks,
@@ -113,17 +111,7 @@ __global__ __launch_bounds__(64 * kEncodeItemTiles) void k_bminmax_prefix(const 
     const uint64_t n = ck.view.n, c = it.c0 + wave;
     const bool mine = c < it.c1;
     int64_t f[16], own = INT64_MAX;
-    if (mine) {
-      uint64_t v[16];
-      const bool full = tile_full(n, c);
-      load_tile_f64(ck.x, n, c, lane, full, v);
-#pragma unroll
-      for (uint32_t g = 0; g < 16; ++g) {
-        f[g] = full || c * kTileRows + 64 * g + lane < n ? fetch_fixed_aligned_bits(v[g], ck.pexp, ck.view.dlen)
-                                                         : INT64_MAX;
-        own = min(own, f[g]);
-      }
-    }
+    if (mine) own = load_tile_fixed(ck.x, n, c, lane, ck.pexp, ck.view.dlen, f);
     own = wave_min_i64(own);
     if (lane == 0) smn[wave] = own;
     int64_t carry = INT64_MAX;
@@ -132,25 +120,7 @@ __global__ __launch_bounds__(64 * kEncodeItemTiles) void k_bminmax_prefix(const 
     __syncthreads();
     for (uint32_t w = 0; w < wave; ++w) carry = min(carry, smn[w]);
     int64_t qmax = INT64_MIN;
-    if (mine) {
-#pragma unroll
-      for (uint32_t g = 0; g < 16; ++g) {
-        int64_t e = carry;
-        if (__any(f[g] < carry)) {
-          int64_t p = f[g];   // min over the lanes up to this one
-#pragma unroll
-          for (uint32_t o = 1; o < 64; o <<= 1) {
-            const int64_t u = (int64_t)__shfl_up((long long)p, o, 64);
-            if (lane >= o) p = min(p, u);
-          }
-          const int64_t u = (int64_t)__shfl_up((long long)p, 1, 64);
-          if (lane) e = min(carry, u);
-          carry = min(carry, (int64_t)__shfl((long long)p, 63, 64));
-        }
-        const bool valid = c * kTileRows + 64 * g + lane < n;
-        if (valid && f[g] >= e) qmax = max(qmax, f[g]);
-      }
-    }
+    if (mine) qmax = lane_prefix_max(f, carry, n - c * kTileRows, lane);
     qmax = wave_max_i64(qmax);
     if (lane == 0) smx[wave] = qmax;
     __syncthreads();

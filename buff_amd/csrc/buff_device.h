@@ -379,6 +379,47 @@ __device__ __forceinline__ void load_tile_f64(const double* __restrict__ x, uint
   }
 }
 
+// The fixed-point values of rows 64g + lane of tile c (INT64_MAX past the end); returns the lane's min.
+__device__ __forceinline__ int64_t load_tile_fixed(const double* __restrict__ x, uint64_t n, uint64_t c, uint32_t lane,
+                                                   int32_t pexp, uint32_t dlen, int64_t (&f)[16]) {
+  uint64_t v[16];
+  const bool full = tile_full(n, c);
+  load_tile_f64(x, n, c, lane, full, v);
+  int64_t mn = INT64_MAX;
+#pragma unroll
+  for (uint32_t g = 0; g < 16; ++g) {
+    f[g] = full || c * kTileRows + 64 * g + lane < n ? fetch_fixed_aligned_bits(v[g], pexp, dlen) : INT64_MAX;
+    mn = min(mn, f[g]);
+  }
+  return mn;
+}
+
+// The lane's max over its rows of the tile f (the first `rows` count) that are
+// not below every row before them; before: the min of the rows before the tile.
+// A group of 64 rows without a new minimum counts as a whole, the others are
+// scanned row by row.
+__device__ __forceinline__ int64_t lane_prefix_max(const int64_t (&f)[16], int64_t before, uint64_t rows,
+                                                   uint32_t lane) {
+  int64_t qmax = INT64_MIN;
+#pragma unroll
+  for (uint32_t g = 0; g < 16; ++g) {
+    int64_t e = before;
+    if (__any(f[g] < before)) {
+      int64_t p = f[g];   // min over the lanes up to this one
+#pragma unroll
+      for (uint32_t o = 1; o < 64; o <<= 1) {
+        const int64_t u = (int64_t)__shfl_up((long long)p, o, 64);
+        if (lane >= o) p = min(p, u);
+      }
+      const int64_t u = (int64_t)__shfl_up((long long)p, 1, 64);
+      if (lane) e = min(before, u);
+      before = min(before, (int64_t)__shfl((long long)p, 63, 64));
+    }
+    if (64 * g + lane < rows && f[g] >= e) qmax = max(qmax, f[g]);
+  }
+  return qmax;
+}
+
 // LDS staging of a tile's 1024 u64/f64 values in row order (one pad slot per 16 rows).
 constexpr uint32_t kLdsRow = 17;  // u64 slots per 16 rows (+1 pad)
 

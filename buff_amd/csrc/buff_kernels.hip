@@ -171,38 +171,44 @@ __global__ __launch_bounds__(256) void k_minmax_final(const double* __restrict__
 // K1b: exact max of the reference's `if fixed<min {..} else if fixed>max {..}`
 // loop (split_double.rs:321-330) for the rare case where row 0 holds the unique
 // maximum: max over rows i with fixed_i >= min(fixed_0..fixed_{i-1})
-// (min of the empty prefix = i64::MAX). One wave per workgroup walks its
-// segment in row order with a wave prefix-min scan.
-__global__ __launch_bounds__(64) void k_minmax_prefix(const double* __restrict__ x, uint64_t n, uint64_t ntiles,
-                                                      uint64_t tpw, int32_t pexp, uint32_t dlen,
-                                                      const int64_t* __restrict__ partial,
-                                                      int64_t* __restrict__ partial2) {
-  const uint32_t lane = __lane_id();
+// (min of the empty prefix = i64::MAX). A workgroup owns a range of k_minmax,
+// a wave a tile of it in turn; the minimum before a wave's tile is the earlier
+// ranges' (partial), the earlier rounds' and the earlier waves'. Bound by the
+// rounds, each a dependent load: with the fold, 1,048,576 rows take 11 us (17
+// where the column falls throughout and every group is scanned) and 4,194,304
+// rows 21 (33); one wave a range, row by row, 42 and 53.
+__global__ __launch_bounds__(256) void k_minmax_prefix(const double* __restrict__ x, uint64_t n, uint64_t ntiles,
+                                                       uint64_t tpw, int32_t pexp, uint32_t dlen,
+                                                       const int64_t* __restrict__ partial,
+                                                       int64_t* __restrict__ partial2) {
+  __shared__ int64_t smn[2][4], smx[4];   // the minima by round parity: a wave can be a round ahead of the slowest
+  const uint32_t lane = __lane_id(), wave = wave_in_wg();
+  const uint64_t t0 = (uint64_t)blockIdx.x * tpw;
+  const uint64_t t1 = min(t0 + tpw, ntiles);
   int64_t carry = INT64_MAX;
   for (uint32_t i = lane; i < blockIdx.x; i += 64) carry = min(carry, partial[i]);
   carry = wave_min_i64(carry);
-  const uint64_t t0 = (uint64_t)blockIdx.x * tpw;
-  const uint64_t t1 = min(t0 + tpw, ntiles);
   int64_t qmax = INT64_MIN;
-  for (uint64_t c = t0; c < t1; ++c) {
-    for (uint32_t g = 0; g < 16; ++g) {
-      const uint64_t row = c * kTileRows + 64 * g + lane;
-      const bool valid = row < n;
-      int64_t f = valid ? fetch_fixed_aligned_bits(__double_as_longlong(x[row]), pexp, dlen) : INT64_MAX;
-      int64_t s = f;   // inclusive prefix min over lanes
-#pragma unroll
-      for (uint32_t o = 1; o < 64; o <<= 1) {
-        int64_t u = (int64_t)__shfl_up((long long)s, o, 64);
-        if (lane >= o) s = min(s, u);
-      }
-      int64_t e = (int64_t)__shfl_up((long long)s, 1, 64);
-      e = lane == 0 ? carry : min(carry, e);
-      if (valid && f >= e) qmax = max(qmax, f);
-      carry = min(carry, (int64_t)__shfl((long long)s, 63, 64));
+  uint32_t par = 0;
+  for (uint64_t base = t0; base < t1; base += 4, par ^= 1u) {
+    const uint64_t c = base + wave;
+    const bool mine = c < t1;
+    int64_t f[16], own = INT64_MAX;
+    if (mine) own = load_tile_fixed(x, n, c, lane, pexp, dlen, f);
+    own = wave_min_i64(own);
+    if (lane == 0) smn[par][wave] = own;
+    __syncthreads();
+    int64_t before = carry;
+    for (uint32_t w = 0; w < 4; ++w) {
+      if (w < wave) before = min(before, smn[par][w]);
+      carry = min(carry, smn[par][w]);
     }
+    if (mine) qmax = max(qmax, lane_prefix_max(f, before, n - c * kTileRows, lane));
   }
   qmax = wave_max_i64(qmax);
-  if (lane == 0) partial2[blockIdx.x] = qmax;
+  if (lane == 0) smx[wave] = qmax;
+  __syncthreads();
+  if (threadIdx.x == 0) partial2[blockIdx.x] = max(max(smx[0], smx[1]), max(smx[2], smx[3]));
 }
 
 __global__ __launch_bounds__(64) void k_minmax_prefix_final(const int64_t* __restrict__ partial2, uint32_t nwg,
@@ -1147,7 +1153,7 @@ hipError_t launch_minmax(const double* x, uint64_t n, int32_t pexp, uint32_t dle
     launch_k(k_minmax_final, dim3(1), dim3(256), 0, s, x, n, pexp, dlen, (const int64_t*)partial, nwg,
                        out);
   } else {
-    launch_k(k_minmax_prefix, dim3(nwg), dim3(64), 0, s, x, n, ntiles, tpw, pexp, dlen,
+    launch_k(k_minmax_prefix, dim3(nwg), dim3(256), 0, s, x, n, ntiles, tpw, pexp, dlen,
                        (const int64_t*)partial, partial2);
     launch_k(k_minmax_prefix_final, dim3(1), dim3(64), 0, s, (const int64_t*)partial2, nwg, out);
   }
