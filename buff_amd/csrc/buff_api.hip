@@ -331,14 +331,17 @@ int Ctx::prof_collect() {
 }
 
 LaunchShape Ctx::shape(Op op, const ChunkView& v) const {
-  auto it = tuned.find(tune_key(op, v.ntiles, v.P));
-  if (it != tuned.end()) return it->second;
-  return default_shape(op, v.ntiles);
+  // sums are tuned as one operation; small ones with their hand-over, which SumRows does not have
+  const bool own = op != Op::SumRows || v.ntiles > kSmallSumTiles;
+  auto it = tuned.find(tune_key(op == Op::SumRows ? Op::Sum : op, v.ntiles, v.P));
+  if (own && it != tuned.end()) return it->second;
+  return default_shape(op, v.ntiles, v.P);
 }
 
-// The shape of an operation that was not tuned, by the column's tiles (times:
-// kernels of walk and uniform columns, as the tuner and a trace give them).
-LaunchShape default_shape(Op op, uint64_t ntiles) {
+// The shape of an operation that was not tuned, by the column's tiles and byte
+// planes (times: kernels of walk and uniform columns, as the tuner and a trace
+// give them).
+LaunchShape default_shape(Op op, uint64_t ntiles, uint32_t planes) {
   switch (op) {
     case Op::FilterGt:
     case Op::FilterEq:
@@ -358,13 +361,23 @@ LaunchShape default_shape(Op op, uint64_t ntiles) {
       // 134M cold 287 -> 266; encode: 17M 32.4 -> 31.4, 67M 133 -> 120)
       return LaunchShape{4, 16384, 0, 0};
     case Op::Sum:
-      // few tiles: at most 64 workgroups, which hand the sums over themselves (a
-      // call on 4097 rows 13.5 -> 11.6 us, on 1M 14.6 -> 14.0; 256 workgroups of one
-      // tile a wave 15.9), then one tile per wave; many: half the resident waves,
-      // whose own loads keep memory busy (134M cold 79.6 -> 70.5)
-      if (ntiles <= 1024) return LaunchShape{4, 64, 4, 0};
-      if (ntiles <= 4096) return LaunchShape{4, 1024, 1, 0};
-      if (ntiles <= 32768) return LaunchShape{4, 1024, 2, 0};
+      // few tiles: four a wave, so at most 64 workgroups, which hand the sums over
+      // themselves (a call on 4097 rows 13.5 -> 11.6 us, on 1M 14.6 -> 14.0; 256
+      // workgroups of one tile a wave 15.9)
+      if (ntiles <= kSmallSumTiles) return LaunchShape{4, 1024, 4, 0};
+      [[fallthrough]];
+    case Op::SumRows:
+      // one tile a wave while the workgroups are few (calls of two launches on 300K
+      // and 700K rows: 16.2 us, 16.9 with the kernel's own two or four tiles, 17.7
+      // with four; 2M rows 15.4, 15.8), then the kernel's own (4M rows of two
+      // planes 14.2 us of a call, of three 16.2; with one 16.1 and 17.0), then two
+      if (ntiles <= 2048) return LaunchShape{4, 1024, 1, 0};
+      if (ntiles <= 4096) return LaunchShape{4, 1024, 0, 0};
+      // Many: half the resident waves, whose own loads keep memory busy, and from
+      // three planes on half of that again (134M rows cold, three planes 88.8 ->
+      // 81.3 us with 1024 workgroups of two waves, 85.6 of four; two planes without
+      // a tail 44.5 -> 49.2 and 41.5, two of 2 tail bits 74.8 -> 71.0 and 73.6)
+      if (ntiles <= 32768 || planes <= 2) return LaunchShape{4, 1024, 2, 0};
       return LaunchShape{2, 1024, 2, 0};
     default:
       return LaunchShape{4, 0, 0, 0};
@@ -1218,7 +1231,7 @@ int sum_precision_op(Ctx* ctx, const Chunk* ch, int32_t precision, uint32_t flag
     pv.P = nplanes;
     pv.r = (q > 0 && q == v.r) ? v.r : 0;
     if (pv.P || pv.r) {
-      const LaunchShape ls = ctx->shape(Op::Sum, pv);
+      const LaunchShape ls = ctx->shape(Op::SumRows, pv);
       BUFF_TRY(ctx->scratch(ctx->s_sums, sizeof(ps) + sum_scratch_bytes(ls)));
       ProfScope sc(ctx, "k_sum");
       HIP_TRY(launch_sum(pv, (unsigned long long*)ctx->s_sums.ptr, ctx->stream, ls));
@@ -1479,7 +1492,7 @@ int tune_chunk(Ctx* ctx, const Chunk* ch, double pred, buff_tune_choice* out) {
     };
     buff_tune_choice ch_out{};
     ch_out.op = (uint32_t)op;
-    LaunchShape best = default_shape(op, v.ntiles);
+    LaunchShape best = default_shape(op, v.ntiles, v.P);
     float best_us = 0;
     rc = measure(best, &best_us);
     ch_out.default_us = best_us;

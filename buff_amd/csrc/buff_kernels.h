@@ -56,6 +56,10 @@ hipError_t launch_publish(const void* src, uint32_t mode, uint32_t nk, const Pub
 // the handover cost a large grid more than a second launch: 72 -> 160 us for a
 // sum of 134M rows); tickets of one address serialize, about 11 ns each.
 constexpr uint32_t kFusedWgs = 256;
+// Sums: the tickets of 128 workgroups (1M rows 14.5 us of a call) cost as much as
+// the launch they save, of 256 more (4M rows of two planes 16.1 us of a call, 14.2
+// with the hand-over as a launch).
+constexpr uint32_t kFusedSumWgs = 128;
 
 // Workgroups of the min/max pass over ntiles tiles (all resident at once).
 uint32_t minmax_grid(uint64_t ntiles);
@@ -105,7 +109,7 @@ hipError_t launch_sum(const ChunkView& cv, unsigned long long* sums, hipStream_t
 // One launch: per-plane sums (and the weighted tail sum at k = P) added into
 // the slot set `set` (u64 [kMaxPlanes + 1][kSumSlots], to be summed over the
 // slots); `next`, the set the following call adds into, is cleared. The first
-// set must be zero. With `pub` and at most kFusedWgs workgroups the launch
+// set must be zero. With `pub` and at most kFusedSumWgs workgroups the launch
 // publishes the sums itself (*published; the set is zero again).
 constexpr uint32_t kSumSlots = 64;
 constexpr uint32_t kSumTicket = (kMaxPlanes + 1) * kSumSlots;   // word of a set

@@ -1340,7 +1340,7 @@ static void launch_sum_pru(const ChunkView& cv, unsigned long long* sums, unsign
       grid_for((cv.ntiles + U - 1) / U, ls.waves_per_wg, cap_of(ls, resident_wgs(k_sum<P, R, U>, block))),
       kMaxSumRows);
   if (next) {
-    const bool fused = pub && wg <= kFusedWgs;
+    const bool fused = pub && wg <= kFusedSumWgs;
     if (published) *published = fused;
     launch_k((k_sum<P, R, U>), dim3(wg), dim3(block), 0, s, cv, sums, next, fused ? *pub : Publish{});
     return;

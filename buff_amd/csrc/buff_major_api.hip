@@ -686,7 +686,7 @@ int major_sum(Ctx* ctx, const Chunk* ch, uint32_t flags, double* ref_sum, double
   const uint32_t S = ch->S;
   uint64_t dense_ps[kMaxPlanes + 1] = {0};
   uint64_t outsum[kMaxSparse] = {0};
-  const LaunchShape ls = ctx->shape(Op::Sum, v);
+  const LaunchShape ls = ctx->shape(Op::SumRows, v);
   // [outlier sums | pad | per-block outlier rows (4 KiB) | dense sums + k_sum rows]
   const uint64_t rows_off = 256, dense_off = rows_off + 4096;
   BUFF_TRY(ctx->scratch(ctx->s_sums, dense_off + sizeof(dense_ps) + sum_scratch_bytes(ls)));
@@ -1050,7 +1050,7 @@ int residue_sum_op(Ctx* ctx, const Chunk* ch, int32_t precision, uint32_t flags,
   uint64_t osum[kMaxSparse] = {0};
   uint64_t fields[2] = {0, 0};
   if (ch->n > 0) {
-    const LaunchShape ls = ctx->shape(Op::Sum, v);
+    const LaunchShape ls = ctx->shape(Op::SumRows, v);
     const uint64_t rows_off = 256, dense_off = rows_off + 4096;
     BUFF_TRY(ctx->scratch(ctx->s_sums, dense_off + sizeof(ps) + sum_scratch_bytes(ls)));
     uint8_t* sb = (uint8_t*)ctx->s_sums.ptr;

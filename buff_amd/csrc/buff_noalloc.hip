@@ -64,7 +64,7 @@ int sum_noalloc(Ctx* ctx, const Chunk* ch, double* ref_sum, double* exact_sum, u
   uint64_t ps[kMaxPlanes + 1] = {0};
   const ChunkView& v = ch->view;
   if (ch->n > 0 && (v.P || v.r)) {
-    const LaunchShape ls = ctx->shape(Op::Sum, v);
+    const LaunchShape ls = ctx->shape(Op::SumRows, v);
     const uint64_t need = sum_scratch_bytes(ls);   // the 9 results, then at most kMaxSumRows rows
     if (need > kNoAllocScratchBytes)
       return fail(BUFF_E_UNSUPPORTED, "the sum needs %llu bytes of scratch, above the %llu of buff_sum_noalloc",

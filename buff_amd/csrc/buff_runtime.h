@@ -39,7 +39,11 @@ uint64_t stream_bytes_of(uint64_t n, uint32_t P, uint32_t r);
 
 inline uint64_t round_up(uint64_t x, uint64_t a) { return (x + a - 1) / a * a; }
 
-enum class Op : uint32_t { Encode = 0, FilterGt, FilterEq, Sum, Max, Materialize, kCount };
+// SumRows: a sum by two launches (k_sum, k_sum_final), whose caller reads the
+// result from device memory; Sum: one that may hand its result over itself.
+enum class Op : uint32_t { Encode = 0, FilterGt, FilterEq, Sum, Max, Materialize, SumRows, kCount };
+// Columns of at most this many tiles: a sum hands its result over itself.
+constexpr uint64_t kSmallSumTiles = 1024;
 
 uint32_t tune_bucket(uint64_t ntiles);
 // Launch shapes are kept per (operation, size class, byte planes).
@@ -47,7 +51,7 @@ inline uint64_t tune_key(Op op, uint64_t ntiles, uint32_t planes) {
   return ((uint64_t)op << 40) | ((uint64_t)planes << 32) | tune_bucket(ntiles);
 }
 
-LaunchShape default_shape(Op op, uint64_t ntiles);
+LaunchShape default_shape(Op op, uint64_t ntiles, uint32_t planes);
 
 struct Scratch {
   void* ptr = nullptr;

@@ -307,3 +307,44 @@ def test_condition_values_largest(ctx, rows):
     got = ch.materialize_cond(words.view(np.uint32)[: (rows + 31) // 32], flags=buff_amd.BUFF_SEMANTIC)
     assert np.array_equal(got, want)
     ch.free()
+
+
+# the sums' launch shapes: by tiles (up to 1024, 2048, 4096, 32768 and more) and planes (one, two, more), with the
+# hand-over in the launch and by two launches
+@pytest.mark.parametrize("decimals,high", [(1, 50), (2, 1000), (4, 1000)])
+@pytest.mark.parametrize("rows", [1024 * TILE, 1024 * TILE + 1, 2048 * TILE, 2048 * TILE + 1, 4096 * TILE + 3,
+                                  32768 * TILE, 32768 * TILE + 1])
+def test_sum(ctx, decimals, high, rows):
+    x = datagen.uniform(rows, -high, high, decimals, rows)
+    x[0] = -high - 1.5
+    ch = ctx.encode(x, 10 ** decimals)
+    info = ch.info()
+    f = fixed(x, info.dlen)
+    want = float(f.sum()) / 2.0 ** info.dlen
+    a, b = ch.sum(), ch.sum_noalloc()
+    assert a[1] == want and b[1] == want and a[0] == b[0] and np.array_equal(a[2], b[2])
+    kept = min(5, info.dlen)   # the fraction bits of one decimal
+    exact = ch.sum_precision(1, flags=buff_amd.BUFF_SEMANTIC)[1]
+    drop = info.dlen - kept
+    assert exact == float((((f - info.base) >> drop << drop) + info.base).sum()) / 2.0 ** info.dlen
+    ch.free()
+
+
+# a narrow column's sum takes the time of its bytes: 13 bits a row against 26
+def test_sum_time(ctx):
+    rows = 1 << 26
+    us = []
+    for decimals, high in ((1, 50), (4, 1000)):
+        x = datagen.uniform(rows, -high, high, decimals, 3)
+        x[0] = -high - 1.5
+        ch = ctx.encode(x, 10 ** decimals)
+        best = np.inf
+        for _ in range(8):
+            ctx.prof_reset()
+            ctx.prof_enable(True)
+            ch.sum()
+            best = min(best, ctx.prof_query("k_sum")[1] * 1e3)
+            ctx.prof_enable(False)
+        us.append(best)
+        ch.free()
+    assert us[0] < 0.65 * us[1], us
