@@ -1412,7 +1412,8 @@ struct OpTimer {
 // Times every candidate shape of the range filter, sum, max and full
 // materialization on this chunk (best of three runs each, the memory-side cache
 // evicted before every run) and keeps the fastest per operation for chunks of
-// the same size class and byte planes.
+// the same size class and byte planes. The max of a small column has one form
+// (k_max_direct): it is timed and reported, and nothing is kept.
 int tune_chunk(Ctx* ctx, const Chunk* ch, double pred, buff_tune_choice* out) {
   if (ch->S > 0 || (ch->flags & BUFF_MAJORITY))
     return fail(BUFF_E_UNSUPPORTED, "launch-shape tuning covers byte_fixed chunks");
@@ -1440,10 +1441,12 @@ int tune_chunk(Ctx* ctx, const Chunk* ch, double pred, buff_tune_choice* out) {
   const uint32_t tiles_opts[4][3] = {{2, 4, 8}, {1, 2, 4}, {4, 8, 16}, {0, 0, 0}};
   for (int oi = 0; oi < 4 && rc == BUFF_OK; ++oi) {
     const Op op = ops[oi];
-    // sums and maxima: every shape's result (handed over as the operations
-    // do) must equal the first (default shape) run's
+    // sums and maxima are timed with their hand-over, as the operations run them
+    // (a small sum's shape decides whether that is a launch of its own), and
+    // every shape's result must equal the first (default shape) run's
     const uint32_t nres = op == Op::Sum ? v.P + 1 : (op == Op::Max ? 1u : 0u);
-    const void* res = nullptr;   // where the last run left its result
+    const bool direct = op == Op::Max && v.ntiles <= kMaxDirectTiles;   // has no shape
+    Publish pub;   // of the last run
     uint64_t want[kMaxPlanes + 1], got[kMaxPlanes + 1];
     bool have_want = false;
     auto run = [&](const LaunchShape& ls) -> hipError_t {
@@ -1453,18 +1456,27 @@ int tune_chunk(Ctx* ctx, const Chunk* ch, double pred, buff_tune_choice* out) {
         case Op::Sum: {
           unsigned long long *set = nullptr, *next = nullptr;
           if (ctx->sum_slots(&set, &next) != BUFF_OK) return hipErrorUnknown;
-          const hipError_t e = launch_sum_slots(v, set, next, ctx->stream, ls);
-          if (e == hipSuccess) ctx->sum_slots_used();
-          res = set;
-          return e;
+          pub = ctx->next_publish();
+          bool fused = false;
+          const hipError_t e = launch_sum_slots(v, set, next, ctx->stream, ls, &pub, &fused);
+          if (e != hipSuccess || fused) return e;
+          ctx->sum_slots_used();
+          return launch_publish(set, kPublishSumSlots, nres, pub, ctx->stream);
         }
         case Op::Max: {
+          if (direct) {
+            unsigned long long *set = nullptr, *next = nullptr;
+            if (ctx->sum_slots(&set, &next) != BUFF_OK) return hipErrorUnknown;
+            pub = ctx->next_publish();
+            return launch_max_direct(v, set, pub, ctx->stream);
+          }
           uint8_t* sb = (uint8_t*)ctx->s_best.ptr;
           unsigned int* slots = nullptr;
           uint32_t tag = 0;
           if (ctx->max_slots(&slots, &tag) != BUFF_OK) return hipErrorUnknown;
-          res = sb;
-          return launch_max(v, (unsigned long long*)sb, sb + 512, slots, tag, ctx->stream, ls);
+          pub = ctx->next_publish();
+          const hipError_t e = launch_max(v, (unsigned long long*)sb, sb + 512, slots, tag, ctx->stream, ls);
+          return e != hipSuccess ? e : launch_publish(sb, kPublishCopy, nres, pub, ctx->stream);
         }
         default:
           return launch_materialize(v, mp, (double*)ctx->s_values.ptr, ctx->stream, ls);
@@ -1478,8 +1490,6 @@ int tune_chunk(Ctx* ctx, const Chunk* ch, double pred, buff_tune_choice* out) {
         BUFF_TRY(tm.time(ctx, [&] { return run(ls); }, &us));
         if (rep > 0) *best_us = std::min(*best_us, us);
         if (nres) {
-          Publish pub;
-          BUFF_TRY(ctx->publish(res, op == Op::Sum ? kPublishSumSlots : kPublishCopy, nres, &pub));
           BUFF_TRY(ctx->published(pub, have_want ? got : want, nres));
           if (have_want && memcmp(got, want, 8ull * nres) != 0)
             return fail(BUFF_E_DEVICE, "tuning: launch shape (%u waves, %u workgroups, %u tiles, form %u) changed "
@@ -1500,7 +1510,7 @@ int tune_chunk(Ctx* ctx, const Chunk* ch, double pred, buff_tune_choice* out) {
       for (uint32_t cap : {0u, 1024u, 2048u, 4096u, 8192u, 16384u}) {
         for (uint32_t t : tiles_opts[oi]) {
           for (uint32_t pf = 0; pf < ((op == Op::FilterGt || op == Op::Max) ? 2u : 1u); ++pf) {
-            if (rc != BUFF_OK) break;
+            if (rc != BUFF_OK || direct) break;
             if (op == Op::Materialize && waves != 4) continue;   // its LDS staging assumes four waves
             const LaunchShape ls{waves, cap, t, pf};
             float us = 0;
@@ -1515,7 +1525,7 @@ int tune_chunk(Ctx* ctx, const Chunk* ch, double pred, buff_tune_choice* out) {
       }
     }
     if (rc != BUFF_OK) break;
-    ctx->tuned[tune_key(op, v.ntiles, v.P)] = best;
+    if (!direct) ctx->tuned[tune_key(op, v.ntiles, v.P)] = best;
     if (op == Op::FilterGt) ctx->tuned[tune_key(Op::FilterEq, v.ntiles, v.P)] = best;
     ch_out.waves_per_wg = best.waves_per_wg;
     ch_out.max_wg = best.max_wg;

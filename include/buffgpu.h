@@ -323,8 +323,8 @@ typedef struct {
   uint32_t prefetch;       /* range filter: next step's top plane loaded before refining; max: 1 = the
                               one-pass form (0: the top bytes of every tile, then only the tiles holding
                               the largest) */
-  float best_us;           /* kernel time of the chosen shape */
-  float default_us;        /* kernel time of the default shape */
+  float best_us;           /* device time of the chosen shape (sum and max: with the hand-over of the result) */
+  float default_us;        /* the same of the default shape (max of up to 1,048,576 rows: its only form) */
 } buff_tune_choice;
 int buff_tune_chunk(buff_ctx* ctx, const buff_chunk* chunk, double pred, buff_tune_choice* choices);
 

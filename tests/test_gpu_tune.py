@@ -57,3 +57,44 @@ def test_tune_rejects_unsupported(gpu_ctx):
             ch.tune(100.0)
     finally:
         ch.free()
+
+
+# a small column's sum and max hand their result over in their own launch: the tuner times them so, and finds no shape
+# for the max (up to 1024 tiles it has one form)
+@pytest.mark.parametrize("rows", [4097, 1 << 20])
+def test_tuned_small_column(rows):
+    import time
+
+    import buff_amd
+
+    def call_us(fn):
+        best = np.inf
+        for _ in range(8):
+            t = time.perf_counter()
+            for _ in range(100):
+                fn()
+            best = min(best, (time.perf_counter() - t) * 1e4)
+        return best
+
+    ctx = buff_amd.Context(0)
+    x = dg.uniform(rows, -1000, 1000, 4, 7)
+    x[0] = -1000.5
+    ch = ctx.encode(x, 10 ** 4)
+    answers = ch.sum()[1], ch.max()
+    before = call_us(ch.sum)
+    choice = ch.tune(float(np.quantile(x, 0.9, method="lower")))
+    assert choice["max"]["best_us"] == choice["max"]["default_us"] and choice["max"]["max_wg"] == 0
+    assert (ch.sum()[1], ch.max()) == answers
+    after = call_us(ch.sum)
+    assert after < 1.09 * before, (before, after, choice["sum"])
+    ch.free()
+    ctx.destroy()
+
+
+def test_tuned_above_small(gpu_ctx, oracle):
+    x = dg.random_walk(1024 * 1024 + 1, 4, 33)
+    ch = gpu_ctx.encode(x, 10 ** 4)
+    choice = ch.tune(float(np.quantile(x, 0.9, method="lower")))
+    assert 0 < choice["max"]["best_us"] <= choice["max"]["default_us"]
+    _check(ch, oracle, x, 10 ** 4)
+    ch.free()
