@@ -794,8 +794,7 @@ int filter_cond_device(Ctx* ctx, const Chunk* ch, int op, double pred, uint32_t 
     return BUFF_OK;
   }
   ProfScope ps(ctx, op == BUFF_OP_GT ? "k_filter_cond_gt" : "k_filter_cond_eq");
-  HIP_TRY(launch_filter_cond(ch->view, op == BUFF_OP_GT ? 0 : 1, tg, cond, words, nwords, ctx->stream,
-                             ctx->shape(op == BUFF_OP_GT ? Op::FilterGt : Op::FilterEq, ch->view)));
+  HIP_TRY(launch_filter_cond(ch->view, op == BUFF_OP_GT ? 0 : 1, tg, cond, words, nwords, ctx->stream));
   return BUFF_OK;
 }
 

@@ -91,7 +91,7 @@ hipError_t launch_bitmap_logic(uint64_t* out, const uint64_t* a, const uint64_t*
                                uint64_t nwords, uint64_t cover, int inv_a, int inv_b, hipStream_t s);
 // Filter restricted to the rows set in `cond` (ceil(n/64) u64 words, the bitmap layout).
 hipError_t launch_filter_cond(const ChunkView& cv, int op, const FilterTarget& tg, const uint64_t* cond,
-                              uint64_t* out, uint64_t nwords, hipStream_t s, const LaunchShape& ls);
+                              uint64_t* out, uint64_t nwords, hipStream_t s);
 // out = cond masked to the n rows (copy = 1) or zeros (copy = 0).
 hipError_t launch_cond_fill(uint64_t* out, const uint64_t* cond, uint64_t nwords, uint64_t n, int copy,
                             hipStream_t s);

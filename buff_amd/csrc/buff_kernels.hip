@@ -1252,21 +1252,24 @@ hipError_t launch_filter(const ChunkView& cv, int op, const FilterTarget& tg, ui
   return hipGetLastError();
 }
 
+template <int MODE>
+static void launch_filter_cond_m(const ChunkView& cv, const FilterTarget& tg, const uint16_t* cond, uint64_t* out,
+                                 uint64_t nwords, hipStream_t s) {
+  // Resident workgroups that loop, at every size: a tile without a condition row
+  // costs next to nothing, so there is little to wait for at the end, and starting
+  // more workgroups costs more than it saves (67M rows of a walk, a fiftieth of
+  // them set: 5.9 us, 8.5 with 16384 workgroups of two waves; of a uniform column
+  // 15.1 and 16.6; half of them set 12.7 and 15.3, 23.0 and 23.7).
+  const uint32_t wg = grid_for((cv.ntiles + 3) / 4, 4, resident_wgs(k_filter<MODE, 4, false, true>, 256));
+  launch_k((k_filter<MODE, 4, false, true>), dim3(wg), dim3(256), 0, s, cv, tg, out, nwords,
+           static_cast<unsigned long long*>(nullptr), cond);
+}
+
 hipError_t launch_filter_cond(const ChunkView& cv, int op, const FilterTarget& tg, const uint64_t* cond,
-                              uint64_t* out, uint64_t nwords, hipStream_t s, const LaunchShape& ls) {
-  const uint32_t block = 64 * ls.waves_per_wg;
+                              uint64_t* out, uint64_t nwords, hipStream_t s) {
   const uint16_t* c16 = reinterpret_cast<const uint16_t*>(cond);
-  if (op == 0) {
-    const uint32_t wg = grid_for((cv.ntiles + 3) / 4, ls.waves_per_wg,
-                                 cap_of(ls, resident_wgs(k_filter<0, 4, false, true>, block)));
-    launch_k((k_filter<0, 4, false, true>), dim3(wg), dim3(block), 0, s, cv, tg, out, nwords,
-             static_cast<unsigned long long*>(nullptr), c16);
-  } else {
-    const uint32_t wg = grid_for((cv.ntiles + 3) / 4, ls.waves_per_wg,
-                                 cap_of(ls, resident_wgs(k_filter<1, 4, false, true>, block)));
-    launch_k((k_filter<1, 4, false, true>), dim3(wg), dim3(block), 0, s, cv, tg, out, nwords,
-             static_cast<unsigned long long*>(nullptr), c16);
-  }
+  if (op == 0) launch_filter_cond_m<0>(cv, tg, c16, out, nwords, s);
+  else launch_filter_cond_m<1>(cv, tg, c16, out, nwords, s);
   return hipGetLastError();
 }
 

@@ -249,9 +249,11 @@ __device__ __forceinline__ void major_filter_group(const MV& mv, const MajorTarg
     }
   }
   // RARE (equality where some sparse byte of the target is not the majority
-  // byte): if the first is not, only that column's outliers can match, and few
-  // tiles hold one that does: 40.4 us for such a value on 67,108,864 rows, 43.3
-  // with every tile deposited. A form of its own: the branch costs the others
+  // byte): if the first is not, only that column's outliers can match, and a
+  // tile without one that does ends here. 67,108,864 rows of three sparse columns:
+  // 37.7 us for the rarest first byte and 43.3 for the commonest (every tile
+  // holds it), without this 42.6 for both; 41.9 where a later byte is not the
+  // majority, without 42.6. A form of its own: the branch costs the others
   // registers (equality with the majority value 42.6 -> 47.8).
   if (RARE && S > 1 && ru.eqm[0] == 0) {
     bool hit = false;

@@ -348,3 +348,45 @@ def test_sum_time(ctx):
         us.append(best)
         ch.free()
     assert us[0] < 0.65 * us[1], us
+
+
+# the filter on a condition's rows: its grid does not follow the plain filter's shapes (up to 8192 tiles, to 32768, more)
+@pytest.mark.parametrize("rows", [TILE + 1, 8192 * TILE, 8192 * TILE + 1, 32768 * TILE, 32768 * TILE + 65])
+def test_condition_filter(ctx, rows):
+    rng = np.random.default_rng(rows)
+    x = rng.integers(-10 ** 5, 10 ** 5, rows) / 100.0
+    x[0] = x.min() - 1.5
+    ch = ctx.encode(x, 100)
+    f = fixed(x, ch.info().dlen)
+    for share in (0.02, 0.9):
+        cond = np.repeat(rng.random((rows + 63) // 64) < share, 64)[:rows]
+        cond[-1] = True
+        words = np.packbits(cond, bitorder="little")
+        words = np.pad(words, (0, -len(words) % 4)).view(np.uint32)
+        for op, hit in (("range", f > f[rows // 2]), ("equal", f == f[rows // 2])):
+            got, count = ch.filter_cond(op, float(x[rows // 2]), words, flags=buff_amd.BUFF_SEMANTIC)
+            assert np.array_equal(bits(got, rows), hit & cond) and count == (hit & cond).sum(), (op, share)
+    ch.free()
+
+
+# twice the tiles, few of them with a condition row: less than half as much again
+def test_condition_filter_time(ctx):
+    us = []
+    for rows in (32768 * TILE, 65536 * TILE):
+        x = datagen.random_walk(rows, 4, 5)
+        ch = ctx.encode(x, 10 ** 4)
+        pred = float(np.quantile(x[::97], 0.9))
+        cond, words = (ctx.alloc(rows // 8) for _ in range(2))
+        ch.filter_device("range", float(np.quantile(x[::97], 0.98)), cond.ptr, flags=buff_amd.BUFF_SEMANTIC)
+        best = np.inf
+        for _ in range(12):
+            ctx.prof_reset()
+            ctx.prof_enable(True)
+            ch.filter_cond_device("range", pred, cond.ptr, words.ptr, flags=buff_amd.BUFF_SEMANTIC)
+            ctx.synchronize()
+            best = min(best, ctx.prof_query("k_filter_cond_gt")[1] * 1e3)
+            ctx.prof_enable(False)
+        us.append(best)
+        for b in (ch, cond, words):
+            b.free()
+    assert us[1] < 1.5 * us[0], us
