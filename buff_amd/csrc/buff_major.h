@@ -99,7 +99,7 @@ hipError_t launch_major_filter(const MajorView& mv, int op, bool semantic, const
 // top F - drop bits (drop = 0: every bit); 2: the true offsets' top F - drop
 // bits as a number (off >> drop), the residue format's reduced-precision read.
 hipError_t launch_major_decode(const MajorView& mv, int mode, uint32_t drop, double inv_scale, double* out,
-                               hipStream_t s, const LaunchShape& ls);
+                               hipStream_t s);
 // sums[j] = sum of the outlier bytes of sparse column j; scratch: major_sum_scratch_bytes().
 uint64_t major_sum_scratch_bytes(uint32_t S);
 hipError_t launch_major_outlier_sums(const MajorView& mv, const uint64_t* n_out, unsigned long long* sums,

@@ -775,8 +775,7 @@ int major_materialize_device(Ctx* ctx, const Chunk* ch, int32_t precision, uint3
   if (r == 0) return BUFF_OK;
   if (!out) return fail(BUFF_E_INVALID, "null output");
   ProfScope sc(ctx, "k_major_decode");
-  HIP_TRY(launch_major_decode(major_view(ch), semantic ? 1 : 0, drop, std::ldexp(1.0, -(int)ch->dlen), out, ctx->stream,
-                              ctx->shape(Op::Materialize, ch->view)));
+  HIP_TRY(launch_major_decode(major_view(ch), semantic ? 1 : 0, drop, std::ldexp(1.0, -(int)ch->dlen), out, ctx->stream));
   return BUFF_OK;
 }
 
@@ -1024,8 +1023,7 @@ int residue_materialize_device(Ctx* ctx, const Chunk* ch, int32_t precision, dou
   if (r == 0) return BUFF_OK;
   if (!out) return fail(BUFF_E_INVALID, "null output");
   ProfScope sc(ctx, "k_major_decode");
-  HIP_TRY(launch_major_decode(major_view(ch), 2, ch->F - rr.R, std::ldexp(1.0, -(int)ch->dlen), out, ctx->stream,
-                              ctx->shape(Op::Materialize, ch->view)));
+  HIP_TRY(launch_major_decode(major_view(ch), 2, ch->F - rr.R, std::ldexp(1.0, -(int)ch->dlen), out, ctx->stream));
   return BUFF_OK;
 }
 
