@@ -351,9 +351,11 @@ LaunchShape default_shape(Op op, uint64_t ntiles, uint32_t planes) {
       if (ntiles <= 8192) return LaunchShape{2, 2048, 2, 1};
       // Many: a group of four tiles a wave, the workgroups beyond the resident
       // ones started as others end, instead of resident ones that loop and wait
-      // for the slowest (134M rows, walk 31.6 -> 26.5, uniform cold 48.0 ->
-      // 42.3; 67M 20.3 -> 18.2). At 17M the resident grid is as fast.
-      if (ntiles > 32768) return LaunchShape{2, 16384, 4, 0};
+      // for the slowest (134M rows, walk 31.6 -> 26.5, uniform cold 48.0 -> 42.3;
+      // 67M 20.3 -> 18.2). From 33M to 50M rows the two are within 3% of each other
+      // over the columns, and a walk with a thousandth of its rows above the
+      // predicate is quicker on the resident grid (33.6M 8.6 and 10.6).
+      if (ntiles > 49152) return LaunchShape{2, 16384, 4, 0};
       return LaunchShape{4, 0, 0, 0};
     case Op::Encode:
     case Op::Materialize:

@@ -390,3 +390,16 @@ def test_condition_filter_time(ctx):
         for b in (ch, cond, words):
             b.free()
     assert us[1] < 1.5 * us[0], us
+
+
+# the filters' grids: resident workgroups up to 49152 tiles, then more of them with a group of tiles a wave
+@pytest.mark.parametrize("rows", [49152 * TILE, 49152 * TILE + 1])
+def test_filter_lines(ctx, rows):
+    x = (np.arange(rows, dtype=np.int64) * 7919 % 200_003 - 100_000) / 100.0
+    x[0] = -1001.5
+    ch = ctx.encode(x, 100)
+    for pred in (999.0, 0.5):
+        for op, want in (("range", x > pred), ("equal", x == pred)):
+            words, count = ch.filter(op, pred, flags=buff_amd.BUFF_SEMANTIC)
+            assert np.array_equal(bits(words, rows), want) and count == want.sum(), (op, pred)
+    ch.free()
