@@ -359,9 +359,12 @@ LaunchShape default_shape(Op op, uint64_t ntiles, uint32_t planes) {
       return LaunchShape{4, 0, 0, 0};
     case Op::Encode:
     case Op::Materialize:
-      // the same (materialize: 17M rows 33.4 -> 32.1 us, 67M cold 141 -> 125,
-      // 134M cold 287 -> 266; encode: 17M 32.4 -> 31.4, 67M 133 -> 120)
-      return LaunchShape{4, 16384, 0, 0};
+      // the same, down to a tile a wave (against 2048 workgroups; materialize: 17M
+      // rows 33.4 -> 32.1 us, 67M cold 141 -> 125, 134M cold 285 -> 252; encode: 17M
+      // 32.4 -> 31.4, 67M 133 -> 120, 134M cold 272 -> 253, two planes 235 -> 224.
+      // Held to 16384 workgroups, where waves loop again, the encodes of 134M rows
+      // are slower than on 2048: 282 and 246)
+      return LaunchShape{4, ntiles <= 65536 ? 16384u : 65536u, 0, 0};
     case Op::Sum:
       // few tiles: four a wave, so at most 64 workgroups, which hand the sums over
       // themselves (a call on 4097 rows 13.5 -> 11.6 us, on 1M 14.6 -> 14.0; 256

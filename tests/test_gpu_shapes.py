@@ -403,3 +403,17 @@ def test_filter_lines(ctx, rows):
             words, count = ch.filter(op, pred, flags=buff_amd.BUFF_SEMANTIC)
             assert np.array_equal(bits(words, rows), want) and count == want.sum(), (op, pred)
     ch.free()
+
+
+# encode and decode: up to 16384 workgroups of four tiles, then a tile a wave; sparse columns loop there
+@pytest.mark.parametrize("layout", [0, buff_amd.BUFF_MAJORITY])
+@pytest.mark.parametrize("rows", [65536 * TILE, 65536 * TILE + 1])
+def test_decode_lines(ctx, layout, rows):
+    x = np.tile(np.random.default_rng(3).integers(-4000, 4000, 999_983) / 8.0, rows // 999_983 + 1)[:rows]
+    if layout:
+        x[::37] = 1e6
+    x[0] = x.min() - 1.5
+    ch = ctx.encode(x, 10 ** 3, flags=layout)
+    assert (ch.info().sparse_cols > 0) == bool(layout)
+    assert np.array_equal(ch.materialize(flags=buff_amd.BUFF_SEMANTIC), x)
+    ch.free()
