@@ -6,7 +6,6 @@ fallback; loading fails loudly when the library is missing.
 """
 import collections.abc
 import ctypes
-import operator
 import os
 import threading
 
@@ -500,44 +499,67 @@ class QueryResults(collections.abc.Sequence):
         return self._res[i]
 
 
-class _BatchChunks(collections.abc.Sequence):
-    """The chunks of a batch, each made when it is first asked for (a batch of hundreds is often only queried)."""
+class _BatchChunks(list):
+    """The chunks of a batch: a list whose items are made when they are first asked for by index (a batch of hundreds is
+    often only queried); whatever else is done with it makes all of them first."""
 
     def __init__(self, ctx, batch, n):
+        super().__init__([None] * n)
         self._ctx = ctx
         self._batch = batch
-        self._chunks = [None] * n
+        self._made = []
+        self._lazy = True
         self._lock = threading.Lock()
 
-    def __len__(self):
-        return len(self._chunks)
-
-    def __getitem__(self, i):
-        if isinstance(i, slice):
-            return [self[k] for k in range(*i.indices(len(self._chunks)))]
-        i = operator.index(i)
-        if self._chunks[i] is None:
-            with self._lock:
-                if self._chunks[i] is None:
+    def _fill(self, indexes):
+        with self._lock:
+            for i in indexes:
+                if list.__getitem__(self, i) is None:
                     h = ctypes.c_void_p()
                     if self._batch is not None:
-                        check(lib().buff_batch_chunk(self._batch, i % len(self._chunks), ctypes.byref(h)))
-                    self._chunks[i] = Chunk(self._ctx, h.value, borrowed=True)
-        return self._chunks[i]
+                        check(lib().buff_batch_chunk(self._batch, i, ctypes.byref(h)))
+                    c = Chunk(self._ctx, h.value, borrowed=True)
+                    self._made.append(c)
+                    list.__setitem__(self, i, c)
 
-    def __add__(self, other):
-        return list(self) + list(other)
+    def _whole(self):
+        if self._lazy:
+            self._fill(range(len(self)))
+            self._lazy = False
+
+    def __getitem__(self, i):
+        if self._lazy:
+            at = range(len(self))[i]   # an index from 0 on, or the slice's; IndexError, TypeError as a list's
+            self._fill(at if isinstance(i, slice) else (at,))
+        return super().__getitem__(i)
 
     def __radd__(self, other):
-        return list(other) + list(self)
+        return other + self[:] if isinstance(other, list) else NotImplemented
+
+    def __reduce_ex__(self, protocol):   # copies are plain lists
+        return list, (self[:],)
 
     def drop(self):
         """The batch goes: its chunks have no handle any more."""
         with self._lock:
             self._batch = None
-            for c in self._chunks:
-                if c is not None:
-                    c.handle = None
+            for c in self._made:
+                c.handle = None
+
+
+def _of_all(name):
+    def method(self, *args, **kw):
+        self._whole()
+        return getattr(list, name)(self, *args, **kw)
+
+    method.__name__ = name
+    return method
+
+
+for _name in ("__iter__", "__reversed__", "__contains__", "__eq__", "__ne__", "__lt__", "__le__", "__gt__", "__ge__",
+              "__add__", "__iadd__", "__mul__", "__rmul__", "__imul__", "__setitem__", "__delitem__", "__repr__",
+              "append", "clear", "copy", "count", "extend", "index", "insert", "pop", "remove", "reverse", "sort"):
+    setattr(_BatchChunks, _name, _of_all(_name))
 
 
 class Batch:
