@@ -992,7 +992,7 @@ int max_range_device(Ctx* ctx, const Chunk* ch, uint64_t s, uint64_t e, uint64_t
     if (argmax && nwords) HIP_TRY(launch_fill_bitmap(argmax, nwords, ch->n, 0, ctx->stream));
     return BUFF_OK;
   }
-  if (W >= kWmaxBlockMin && W <= kWmaxBlockMax) {
+  if (wmax_block_form(v, s, e, W)) {
     ProfScope ps(ctx, "k_wmax");
     HIP_TRY(launch_wmax_block(v, s, e, W, k, std::ldexp(1.0, -(int)ch->dlen), vals, want, argmax, ctx->stream));
     return BUFF_OK;

@@ -11,10 +11,11 @@ namespace buffgpu {
 // launch without scratch: the first k maxima to vals, and (argmax not null)
 // ceil(n/64) u64 words of the rows equal to their window's max (want = false:
 // all zero). From 16 rows on a lane's 16 rows hold at most two windows; above
-// 8192 the rows read beyond a workgroup's own 16 tiles (W on average) cost as
-// much as the general path's second read.
+// 8192 the maxima of a workgroup's windows outgrow its own 16 tiles.
 constexpr uint64_t kWmaxBlockMin = 16, kWmaxBlockMax = 8192;
 constexpr uint64_t kWmaxSmallTiles = 2048;   // up to here a wave takes one tile, not four
+// Whether this launch is the quicker form for rows [s, e).
+bool wmax_block_form(const ChunkView& cv, uint64_t s, uint64_t e, uint64_t W);
 hipError_t launch_wmax_block(const ChunkView& cv, uint64_t s, uint64_t e, uint64_t W, uint64_t k, double inv_scale,
                              double* vals, bool want, uint64_t* argmax, hipStream_t st);
 

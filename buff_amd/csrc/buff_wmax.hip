@@ -5,7 +5,7 @@
 // the running max byte, then narrows them plane by plane; the result is each
 // window's max offset. Here every tile of [s, e) is read once and every window
 // segment it holds reduced. Windows of kWmaxBlockMin .. kWmaxBlockMax rows take
-// one launch:
+// one launch (but for the longest on large columns, wmax_block_form):
 //   k_wmax_block   a workgroup holds consecutive tiles in registers, completes
 //                  their windows' maxima in LDS (the rows of its first and last
 //                  window outside its tiles are read too), then compares its
@@ -78,7 +78,7 @@ __global__ __launch_bounds__(64) void k_wmax_tiles(ChunkView cv, uint64_t s, uin
   }
 }
 
-// Windows of more than kWmaxBlockMax rows: a tile holds at most two window
+// Windows of at least one tile (W >= 1024): a tile holds at most two window
 // segments, so each lane keeps its rows' max for both and the wave reduces
 // them; no LDS. One wave per tile, four per workgroup.
 template <int NP>
@@ -395,7 +395,7 @@ static hipError_t launch_wmax_np(const ChunkView& cv, uint64_t s, uint64_t e, ui
   uint32_t* kb[2] = {reinterpret_cast<uint32_t*>(scratch + L.k[0]), reinterpret_cast<uint32_t*>(scratch + L.k[1])};
   unsigned long long* vb[2] = {reinterpret_cast<unsigned long long*>(scratch + L.v[0]),
                                reinterpret_cast<unsigned long long*>(scratch + L.v[1])};
-  if (W > kWmaxBlockMax)
+  if (W >= kTileRows)
     launch_k(k_wmax_tiles_wide<NP>, dim3((uint32_t)((L.ntiles + 3) / 4)), dim3(256), 0, st, cv, s, e, W, L.t_first,
              L.ntiles, wmax, kb[0], vb[0]);
   else
@@ -431,6 +431,25 @@ static void launch_wmax_block_np(const ChunkView& cv, uint64_t s, uint64_t e, ui
   else
     launch_k((k_wmax_block<NP, 4>), dim3((uint32_t)((nt + 4 * kWmaxWaves - 1) / (4 * kWmaxWaves))),
              dim3(64 * kWmaxWaves), 0, st, cv, s, e, W, magic, t0, k, inv_scale, vals, w, o16, nout16);
+}
+
+// The rows read beyond a workgroup's own tiles (W on average; none where the
+// windows' starts divide its 16 tiles) are further dependent loads, and with
+// 64-bit keys (four planes and more) a CU holds half the waves to hide them: the
+// launches that read everything twice, but stream, catch up the sooner the larger
+// the column and the fewer its planes. 134,217,728 rows of four planes, us in one
+// launch and in six: W = 1000 227 and 259, 2047 234 and 234, 7001 291 and 230, 4096
+// 185 and 228; 16,777,216 rows at 7001 42 and 45; 134,217,728 rows of six planes at
+// 7001 284 and 298. Three planes and fewer: at most 0.77 of the six everywhere.
+// Columns of one tile a wave (four in a workgroup, so that at W = 8192 they read
+// three times their rows): 7 us and 23 for 2,097,152 rows of four planes.
+bool wmax_block_form(const ChunkView& cv, uint64_t s, uint64_t e, uint64_t W) {
+  if (W < kWmaxBlockMin || W > kWmaxBlockMax) return false;
+  constexpr uint64_t kOwnRows = 16 * kTileRows;
+  if (cv.P <= 3 || (s % kOwnRows == 0 && kOwnRows % W == 0)) return true;
+  uint64_t most = cv.P == 4 ? 1536 : cv.P == 5 ? 2560 : 5120;
+  for (uint64_t tiles = (e - s + kTileRows - 1) / kTileRows; tiles <= 65536 && most < kWmaxBlockMax; tiles *= 2) most *= 2;
+  return W <= most;
 }
 
 hipError_t launch_wmax_block(const ChunkView& cv, uint64_t s, uint64_t e, uint64_t W, uint64_t k, double inv_scale,

@@ -417,3 +417,45 @@ def test_decode_lines(ctx, layout, rows):
     assert (ch.info().sparse_cols > 0) == bool(layout)
     assert np.array_equal(ch.materialize(flags=buff_amd.BUFF_SEMANTIC), x)
     ch.free()
+
+
+# windowed maxima on columns of four planes: the longest windows of the one-launch form at a size, one row more, and
+# windows that divide its 16 tiles
+@pytest.mark.parametrize("rows,windows", [(16385 * TILE, (6144, 6145, 8192)), (65537 * TILE, (1536, 1537, 4096))])
+def test_windowed_max_lines(ctx, rows, windows):
+    x = datagen.random_walk(rows, 6, 23)
+    ch = ctx.encode(x, 10 ** 6)
+    info = ch.info()
+    assert info.planes == 4
+    f = fixed(x, info.dlen)
+    for window in windows:
+        for s in (0, 17):
+            vals, words = ch.max_range(s, rows, window, flags=buff_amd.BUFF_SEMANTIC)
+            want = np.maximum.reduceat(f[s:], np.arange(0, rows - s, window))
+            assert np.array_equal(vals, want / 2.0 ** info.dlen), (window, s)
+            hit = np.zeros(rows, dtype=bool)
+            hit[s:] = f[s:] == np.repeat(want, window)[: rows - s]
+            assert np.array_equal(bits(words, rows), hit), (window, s)
+    ch.free()
+
+
+# windows of 7001 rows against 1000 on a large column of four planes: the halo of the one-launch form is not read
+def test_windowed_max_time(ctx):
+    rows = 1 << 27
+    x = datagen.random_walk(rows, 6, 23)
+    ch = ctx.encode(x, 10 ** 6)
+    vals, words = ctx.alloc(8 * (rows // 1000 + 1)), ctx.alloc(rows // 8)
+    us = []
+    for window in (1000, 7001):
+        best = np.inf
+        for _ in range(6):
+            ctx.prof_reset()
+            ctx.prof_enable(True)
+            ch.max_range_device(0, rows, window, vals.ptr, rows // 1000 + 1, words.ptr, flags=buff_amd.BUFF_SEMANTIC)
+            ctx.synchronize()
+            best = min(best, ctx.prof_query("k_wmax")[1] * 1e3)
+            ctx.prof_enable(False)
+        us.append(best)
+    for b in (ch, vals, words):
+        b.free()
+    assert us[1] < 1.17 * us[0], us
