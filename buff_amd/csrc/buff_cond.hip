@@ -172,7 +172,7 @@ static CondLayout cond_layout(uint64_t ntiles) {
 // One wave per workgroup range (one tile per lane): the tiles holding
 // condition rows, compacted in tile order, each with its first output row. Up
 // to kCondSelf ranges (SELF) a wave adds up the counts of the ranges before its
-// own, sixteen loads in flight together, and the last one writes the totals: a
+// own, eight loads in flight together, and the last one writes the totals: a
 // scan launch less (a call with next to no hits, 16M / 67M / 134M / 268M rows:
 // 16.7 / 17.9 / 20.4 / 25.5 us, with the scan 19.7 / 20.6 / 23.4 / 29.9 us).
 // Beyond, the reads grow with the square of the ranges and the scan takes over.
