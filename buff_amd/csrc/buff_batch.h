@@ -104,7 +104,7 @@ struct BatchBuffers {
   BItem* items;                      // written by the batch's first kernel
   uint8_t* tile_top;                 // max: per-tile top byte
   unsigned long long* item_acc;      // per item: kMaxPlanes + 1 u64
-  BResult* res;                      // maxima: v[0] the max offset, v[1] the top byte
+  BResult* res;                      // maxima: v[1] the top byte
 };
 
 // `grid` is the persistent grid size and `tiles_per_item` the work item length

@@ -190,13 +190,14 @@ hipError_t launch_batch_encode(const BEncChunk* chunks, const BItem* items, uint
 //   k_bq_scan   items [0, nscan): filters write tile bitmaps and count them,
 //               sums add the sub-column bytes and tail bits, maxima record every
 //               tile's top byte;
-//   k_bq_reduce one wave per query folds its items' partials and writes the
-//               result to pinned host memory;
-//   k_bq_max_refine the tiles holding a max query's top byte give its max offset;
+//   k_bq_reduce folds every query's items' partials and writes the result to
+//               pinned host memory;
+//   k_bq_max_refine the tiles holding a max query's top byte give its items' max
+//               offsets;
 //   k_bq_mat    items [nscan, nitems): materializations, staged through LDS for
 //               coalesced f64 stores (kept apart so the scan kernel holds no LDS
 //               and runs at full occupancy);
-//   k_bq_max_publish writes the maxima to pinned host memory.
+//   k_bq_max_publish folds them and writes the maxima to pinned host memory.
 // Per-tile loads are issued together: a filter reads the top byte plane, then
 // every remaining plane and tail bit-plane of the tied rows at once; sums and
 // materializations read all their planes before combining them.
@@ -498,66 +499,104 @@ __global__ __launch_bounds__(256) void k_bq_fetch(const BatchBuffers* __restrict
   }
 }
 
-// One wave per query folds its items' partials (filters: count, sums:
-// sub-column sums, maxima: the top byte), four partial rows in flight per lane,
-// and writes the result words to pinned host memory, visible to the host once
-// the batch's completion event has fired; a max query's top byte goes to device
-// memory for the refinement. Materializations have nothing to fold. (A
-// workgroup per query with its barriers and a separate copy of every result
-// took 29 + 11 us for 4096 queries.)
-__global__ __launch_bounds__(256) void k_bq_reduce(const BatchBuffers* __restrict__ bbp) {
-  const BatchBuffers bb = cload(bbp);
+// The partials of items first, first + stride, ... of a query, result word k in
+// lane k; four partial rows in flight per lane.
+__device__ __forceinline__ unsigned long long fold_items(const BUFF_GLOBAL unsigned long long* acc, uint32_t nitems,
+                                                         uint32_t first, uint32_t stride, uint32_t nk, bool is_max,
+                                                         uint32_t lane) {
+  unsigned long long v[kMaxPlanes + 1];
+#pragma unroll
+  for (uint32_t k = 0; k <= kMaxPlanes; ++k) v[k] = 0;
+  for (uint32_t i0 = first; i0 < nitems; i0 += 4 * stride) {
+#pragma unroll
+    for (uint32_t k = 0; k <= kMaxPlanes; ++k) {
+      if (k >= nk) continue;
+      unsigned long long a[4];
+#pragma unroll
+      for (uint32_t u = 0; u < 4; ++u) {
+        const uint32_t i = i0 + u * stride;
+        a[u] = i < nitems ? acc[(uint64_t)i * (kMaxPlanes + 1) + k] : 0ull;
+      }
+#pragma unroll
+      for (uint32_t u = 0; u < 4; ++u) v[k] = is_max ? max(v[k], a[u]) : v[k] + a[u];
+    }
+  }
+  unsigned long long mine = 0;
+#pragma unroll
+  for (uint32_t k = 0; k <= kMaxPlanes; ++k) {
+    if (k >= nk) continue;
+    const unsigned long long t = is_max ? wave_max_u64(v[k]) : wave_sum_u64(v[k]);
+    if (lane == k) mine = t;
+  }
+  return mine;
+}
+
+// Folds words word0, word0 + 1, ... of the partials of every query's items: words
+// of the query's operation (0: not folded here), then store(query, operation,
+// words, lane k: word k). One wave a query; a query of more than kWaveItems items,
+// of which a batch holds few, takes a workgroup (two sums over 67M rows have 8192
+// items each: 185 -> 130 us of a call).
+constexpr uint32_t kWaveItems = 512;
+template <typename Words, typename Store>
+__device__ __forceinline__ void fold_queries(const BatchBuffers& bb, uint32_t word0, Words words, Store store) {
+  __shared__ unsigned long long s_part[4][kMaxPlanes + 1];
   const WaveSlot ws = wave_slot();
   const uint32_t lane = ws.lane;
   const uint32_t nq = cmem(bb.hdr)->nq;
   for (uint32_t qi = ws.first; qi < nq; qi += ws.stride) {
     const BUFF_CONST BQuery* q = cmem(bb.q + qi);
-    const uint32_t op = q->op, item0 = q->item0, nitems = q->nitems;
-    if (op == kBqMat) continue;
-    const bool is_max = op == kBqMax;
-    const uint32_t nk = op == kBqSum ? kMaxPlanes + 1 : 1u;
-    const BUFF_GLOBAL unsigned long long* acc = gmem(bb.item_acc) + (uint64_t)item0 * (kMaxPlanes + 1);
-    unsigned long long v[kMaxPlanes + 1];
-#pragma unroll
-    for (uint32_t k = 0; k <= kMaxPlanes; ++k) v[k] = 0;
-    for (uint32_t i0 = lane; i0 < nitems; i0 += 4 * 64) {
-#pragma unroll
-      for (uint32_t k = 0; k <= kMaxPlanes; ++k) {
-        if (k >= nk) continue;
-        unsigned long long a[4];
-#pragma unroll
-        for (uint32_t u = 0; u < 4; ++u) {
-          const uint32_t i = i0 + u * 64;
-          a[u] = i < nitems ? acc[(uint64_t)i * (kMaxPlanes + 1) + k] : 0ull;
-        }
-#pragma unroll
-        for (uint32_t u = 0; u < 4; ++u) v[k] = is_max ? max(v[k], a[u]) : v[k] + a[u];
-      }
-    }
-    unsigned long long mine = 0;   // lane k: result word k
-#pragma unroll
-    for (uint32_t k = 0; k <= kMaxPlanes; ++k) {
-      if (k >= nk) continue;
-      const unsigned long long t = is_max ? wave_max_u64(v[k]) : wave_sum_u64(v[k]);
-      if (lane == k) mine = t;
-    }
-    if (is_max) {
-      // v[1] = the top byte; v[0] is raised by the refinement (a query without
-      // items has none: its result is the 0 written here)
-      if (lane == 0) {
-        bb.res[qi].v[0] = 0;
-        bb.res[qi].v[1] = mine;
-        gmem_w(bb.host_res[qi].v)[0] = 0;
-      }
-    } else if (lane < nk) {
-      gmem_w(bb.host_res[qi].v)[lane] = mine;
-    }
+    const uint32_t op = q->op, nitems = q->nitems, nk = words(op);
+    if (nk == 0 || nitems > kWaveItems) continue;
+    const BUFF_GLOBAL unsigned long long* acc = gmem(bb.item_acc) + (uint64_t)q->item0 * (kMaxPlanes + 1) + word0;
+    store(qi, op, nk, fold_items(acc, nitems, lane, 64, nk, op == kBqMax, lane));
   }
+  for (uint32_t qi = blockIdx.x; qi < nq; qi += gridDim.x) {
+    const BUFF_CONST BQuery* q = cmem(bb.q + qi);
+    const uint32_t op = q->op, nitems = q->nitems, nk = words(op);
+    if (nk == 0 || nitems <= kWaveItems) continue;   // the same for the whole workgroup
+    const BUFF_GLOBAL unsigned long long* acc = gmem(bb.item_acc) + (uint64_t)q->item0 * (kMaxPlanes + 1) + word0;
+    const unsigned long long mine = fold_items(acc, nitems, threadIdx.x, blockDim.x, nk, op == kBqMax, lane);
+    if (lane < nk) s_part[ws.local][lane] = mine;
+    __syncthreads();
+    if (ws.local == 0) {
+      unsigned long long t = 0;
+      if (lane < nk)
+        for (uint32_t w = 0; w < 4; ++w) t = op == kBqMax ? max(t, s_part[w][lane]) : t + s_part[w][lane];
+      store(qi, op, nk, t);
+    }
+    __syncthreads();
+  }
+}
+
+// Folds the items' partials (filters: count, sums: sub-column sums, maxima: the
+// top byte) and writes the result words to pinned host memory, visible to the
+// host once the batch's completion event has fired; a max query's top byte goes
+// to device memory for the refinement. Materializations have nothing to fold. (A
+// workgroup per query with its barriers and a separate copy of every result
+// took 29 + 11 us for 4096 queries.)
+__global__ __launch_bounds__(256) void k_bq_reduce(const BatchBuffers* __restrict__ bbp) {
+  const BatchBuffers bb = cload(bbp);
+  const uint32_t lane = __lane_id();
+  fold_queries(
+      bb, 0, [](uint32_t op) { return op == kBqMat ? 0u : op == kBqSum ? kMaxPlanes + 1 : 1u; },
+      [&](uint32_t qi, uint32_t op, uint32_t nk, unsigned long long mine) {
+        if (op == kBqMax) {
+          if (lane == 0) {
+            bb.res[qi].v[1] = mine;
+            gmem_w(bb.host_res[qi].v)[0] = 0;   // the result of a query without items
+          }
+        } else if (lane < nk) {
+          gmem_w(bb.host_res[qi].v)[lane] = mine;
+        }
+      });
 }
 
 // Maxima: tiles whose top byte equals the query's top byte give the max offset.
 // A wave probes 64 tiles of its item at once and rebuilds the ones that hold
-// the top byte, all planes of a tile in flight together.
+// the top byte, all planes of a tile in flight together. The items' maxima are
+// folded by k_bq_max_publish: raised by atomics, all items of a large chunk whose
+// tiles hold the top byte queue on one address (4M rows of a uniform column: 4096
+// of them, 92 us of a call, 47 so).
 __global__ __launch_bounds__(256) void k_bq_max_refine(const BatchBuffers* __restrict__ bbp) {
   const BatchBuffers bb = cload(bbp);
   const WaveSlot ws = wave_slot();
@@ -581,15 +620,18 @@ __global__ __launch_bounds__(256) void k_bq_max_refine(const BatchBuffers* __res
       }
     }
     best = wave_max_u64(best);
-    if (lane == 0 && best) atomicMax(&bb.res[it.owner].v[0], (unsigned long long)best);
+    if (lane == 0) gmem_w(bb.item_acc)[(uint64_t)i * (kMaxPlanes + 1) + 1] = best;
   }
 }
 
 __global__ __launch_bounds__(256) void k_bq_max_publish(const BatchBuffers* __restrict__ bbp) {
   const BatchBuffers bb = cload(bbp);
-  const uint32_t nq = cmem(bb.hdr)->nq;
-  for (uint32_t qi = blockIdx.x * blockDim.x + threadIdx.x; qi < nq; qi += gridDim.x * blockDim.x)
-    if (gmem(&bb.q[qi].op)[0] == kBqMax) gmem_w(bb.host_res[qi].v)[0] = gmem(bb.res[qi].v)[0];
+  const uint32_t lane = __lane_id();
+  fold_queries(
+      bb, 1, [](uint32_t op) { return op == kBqMax ? 1u : 0u; },
+      [&](uint32_t qi, uint32_t, uint32_t, unsigned long long mine) {
+        if (lane == 0) gmem_w(bb.host_res[qi].v)[0] = mine;
+      });
 }
 
 // Materialize one tile from the top NP planes and mp.tail_bits tail bits below
@@ -886,7 +928,7 @@ hipError_t launch_batch_queries(const BatchBuffers* bb, const BatchTuning& tu, u
   hipLaunchKernelGGL(k_bq_reduce, dim3(1024), dim3(256), 0, s, bb);   // also the results of queries without tiles
   if (parts & kBqPartMax) {
     hipLaunchKernelGGL(k_bq_max_refine, dim3(tu.grid < 2048 ? tu.grid : 2048), dim3(256), 0, s, bb);
-    hipLaunchKernelGGL(k_bq_max_publish, dim3(16), dim3(256), 0, s, bb);
+    hipLaunchKernelGGL(k_bq_max_publish, dim3(256), dim3(256), 0, s, bb);
   }
   const uint32_t mat_grid = tu.grid < kMatGrid ? tu.grid : kMatGrid;
   if (parts & kBqPartMat) hipLaunchKernelGGL(k_bq_mat, dim3(mat_grid), dim3(256), 0, s, bb);

@@ -459,3 +459,55 @@ def test_windowed_max_time(ctx):
     for b in (ch, vals, words):
         b.free()
     assert us[1] < 1.17 * us[0], us
+
+
+def batch_of(ctx, cols, scale):
+    off = np.concatenate([[0], np.cumsum([len(c) for c in cols])]).astype(np.uint64)
+    xd = ctx.alloc(8 * int(off[-1]))
+    xd.upload(np.concatenate(cols))
+    b = ctx.batch_encode_device(xd.ptr, off, np.full(len(cols), scale, dtype=np.uint64))
+    xd.free()
+    return b
+
+
+# batched queries of as many work items as a wave folds, one more, and thousands (a workgroup folds them), beside small ones
+@pytest.mark.parametrize("tiles", [511, 512, 513, 4096])
+def test_batch_fold(ctx, tiles):
+    cols = [datagen.uniform(n, -1000, 1000, 3, 5 + n) for n in (tiles * TILE, 40, 70_000)]
+    for c in cols:
+        c[0] = -1001.5
+    b = batch_of(ctx, cols, 1000)
+    f = [fixed(c, 11) for c in cols]
+    for chunks in ((0,), (0, 1, 2), (1, 0, 2, 0, 1)):
+        qs = [(op, k, 250.0, -1, N.BUFF_SEMANTIC) for op in (N.BUFF_Q_SUM, N.BUFF_Q_MAX, N.BUFF_Q_GT) for k in chunks]
+        for part in (qs, qs[len(chunks): 2 * len(chunks)]):   # all of them, the maxima alone
+            for (op, k, *_), r in zip(part, b.query(part)):
+                if op == N.BUFF_Q_SUM:
+                    assert r.exact == float(f[k].sum()) / 2.0 ** 11
+                elif op == N.BUFF_Q_MAX:
+                    assert r.value == f[k].max() / 2.0 ** 11
+                else:
+                    assert r.count == (f[k] > fixed(250.0, 11)).sum()
+    b.free()
+
+
+# one query on a large chunk has thousands of items: folding them takes little beside the scan
+def test_batch_fold_time(ctx):
+    import time
+
+    x = datagen.uniform(1 << 24, -1000, 1000, 4, 3)
+    x[0] = -1001.5
+    us = {}
+    for op, rows in ((N.BUFF_Q_GT, 1 << 24), (N.BUFF_Q_SUM, 1 << 24), (N.BUFF_Q_SUM, 1 << 22), (N.BUFF_Q_MAX, 1 << 22)):
+        # every tile holds the top byte: the max is refined everywhere
+        b = batch_of(ctx, [x[:rows]], 10 ** 4)
+        q = N.prepare_queries([(op, 0, 100.0, -1, N.BUFF_SEMANTIC)])
+        best = np.inf
+        for _ in range(60):
+            t = time.perf_counter()
+            b.query(q)
+            best = min(best, (time.perf_counter() - t) * 1e6)
+        us[op, rows] = best
+        b.free()
+    assert us[N.BUFF_Q_SUM, 1 << 24] < 1.5 * us[N.BUFF_Q_GT, 1 << 24], us
+    assert us[N.BUFF_Q_MAX, 1 << 22] < 1.2 * us[N.BUFF_Q_SUM, 1 << 22], us
