@@ -201,7 +201,7 @@ __global__ __launch_bounds__(256) void k_major_place(MajorEnc me, uint64_t ntile
 // masks / tile prefixes / first dense plane, then the outlier windows, then the
 // candidates' later planes and tail. S (sparse columns) is a template argument so
 // the per-column state stays in registers.
-template <int MODE, int S, int U, bool PF>
+template <int MODE, int S, int U, bool PF, bool STEP>
 __global__ __launch_bounds__(256) void k_major_filter(MajorPrefix<S> mv, MajorTarget tg, uint32_t sem,
                                                       uint64_t* __restrict__ out, uint64_t nwords) {
   __shared__ unsigned long long s_dep[4][dep_words(S, U)];
@@ -217,7 +217,7 @@ __global__ __launch_bounds__(256) void k_major_filter(MajorPrefix<S> mv, MajorTa
   for (uint64_t grp = wave; grp < ngroups; grp += nwaves) {
     const uint64_t c0 = grp * U;
     uint32_t res[U];
-    major_filter_group<MODE, S, U, PF, MODE == 1 && !PF>(mv, tg, ru, c0, lane, dep, res);
+    major_filter_group<MODE, S, U, PF, STEP>(mv, tg, ru, c0, lane, dep, res);
 #pragma unroll
     for (int u = 0; u < U; ++u) {
       const uint64_t c = c0 + u;
@@ -805,29 +805,31 @@ static uint32_t resident_wgs(K k) {
   return 0;
 }
 
-template <int MODE, int S, bool PF>
+template <int MODE, int S, bool PF, bool STEP>
 static void launch_filter_pf(const MajorView& mv, bool semantic, const MajorTarget& tg, uint64_t* out,
                              uint64_t nwords, hipStream_t s, uint32_t max_wg) {
   constexpr int U = 2;
   const uint64_t groups = (mv.dense.ntiles + U - 1) / U;
-  static const uint32_t fit = resident_wgs(k_major_filter<MODE, S, U, PF>);   // once per kernel
+  static const uint32_t fit = resident_wgs(k_major_filter<MODE, S, U, PF, STEP>);   // once per kernel
   const uint32_t grid = tiles_grid(groups, fit ? std::min(max_wg, fit) : max_wg);
   MajorPrefix<S> pv;   // the columns in use only: a kernel argument lives in scalar registers
   pv.dense = mv.dense;
   for (int j = 0; j < S; ++j) pv.col[j] = mv.col[j];
-  launch_k((k_major_filter<MODE, S, U, PF>), dim3(grid), dim3(256), 0, s, pv, tg, semantic ? 1u : 0u, out, nwords);
+  launch_k((k_major_filter<MODE, S, U, PF, STEP>), dim3(grid), dim3(256), 0, s, pv, tg, semantic ? 1u : 0u, out,
+           nwords);
 }
 
 template <int MODE, int S>
 static void launch_filter_s(const MajorView& mv, bool semantic, const MajorTarget& tg, uint64_t* out,
                             uint64_t nwords, hipStream_t s, uint32_t max_wg) {
-  // the target's sparse bytes all majority bytes: most rows reach the dense planes
-  bool pf = mv.dense.P >= 2;
-  for (uint32_t j = 0; j < mv.S; ++j) pf = pf && tg.digit[j] == mv.col[j].major;
-  if (pf)
-    launch_filter_pf<MODE, S, true>(mv, semantic, tg, out, nwords, s, max_wg);
+  bool major = true;   // the target's sparse bytes are all majority bytes: most rows reach the dense planes
+  for (uint32_t j = 0; j < mv.S; ++j) major = major && tg.digit[j] == mv.col[j].major;
+  if (major && mv.dense.P >= 2)
+    launch_filter_pf<MODE, S, true, false>(mv, semantic, tg, out, nwords, s, max_wg);
+  else if (MODE == 0 || major)
+    launch_filter_pf<MODE, S, false, false>(mv, semantic, tg, out, nwords, s, max_wg);
   else
-    launch_filter_pf<MODE, S, false>(mv, semantic, tg, out, nwords, s, max_wg);
+    launch_filter_pf<MODE, S, false, MODE == 1>(mv, semantic, tg, out, nwords, s, max_wg);
 }
 
 template <int MODE>

@@ -214,9 +214,16 @@ __device__ __forceinline__ MajorRules<S> major_rules(const MV& mv, const MajorTa
 // candidates into the dense planes): the second dense plane and a tail of at
 // most kPfTail bits are loaded in the first round as well, in full, instead of
 // for the candidates' lines in later dependent rounds.
+//
+// STEP (equality with a target of which some sparse byte is not the majority
+// byte): one column a phase, ending with the first that leaves no candidate,
+// since only outliers match such a byte. 67,108,864 rows of three sparse columns
+// with 5% outliers: 40.4 us, 43.2 with the columns in one phase (38.4 and 43 for
+// the rarest first byte); with 9%, where a tile's further outliers are loaded per
+// phase, 51.5 and 63.2.
 constexpr uint32_t kPfTail = 2;
 
-template <int MODE, int S, int U, bool PF = false, bool RARE = false, typename MV>
+template <int MODE, int S, int U, bool PF = false, bool STEP = false, typename MV>
 __device__ __forceinline__ void major_filter_group(const MV& mv, const MajorTarget& tg, const MajorRules<S>& ru,
                                                    uint64_t c0, uint32_t lane, unsigned long long* dep,
                                                    uint32_t (&res)[U]) {
@@ -248,35 +255,15 @@ __device__ __forceinline__ void major_filter_group(const MV& mv, const MajorTarg
       byte0[u][j] = has ? mv.col[j].outl[p0[u][j] + lane] : 0u;
     }
   }
-  // RARE (equality where some sparse byte of the target is not the majority
-  // byte): if the first is not, only that column's outliers can match, and a
-  // tile without one that does ends here. 67,108,864 rows of three sparse columns:
-  // 37.7 us for the rarest first byte and 43.3 for the commonest (every tile
-  // holds it), without this 42.6 for both; 41.9 where a later byte is not the
-  // majority, without 42.6. A form of its own: the branch costs the others
-  // registers (equality with the majority value 42.6 -> 47.8).
-  if (RARE && S > 1 && ru.eqm[0] == 0) {
-    bool hit = false;
-#pragma unroll
-    for (int u = 0; u < U; ++u) {
-      hit |= lane < cnt[u][0] && byte0[u][0] == tg.digit[0];
-      for (uint32_t k = lane + 64; k < cnt[u][0]; k += 64) hit |= mv.col[0].outl[p0[u][0] + k] == tg.digit[0];
-    }
-    if (__ballot(hit) == 0) {
-#pragma unroll
-      for (int u = 0; u < U; ++u) res[u] = 0;
-      return;
-    }
-  }
   uint32_t cand[U];
 #pragma unroll
   for (int u = 0; u < U; ++u) {
     res[u] = 0;
     cand[u] = tile_full(dv.n, c0 + u) ? 0xFFFFu : lane_valid16(dv.n, c0 + u, lane);
   }
+  constexpr int N = STEP ? 1 : S < kDepCols ? S : kDepCols;   // words per lane and tile
 #pragma unroll
-  for (int jp = 0; jp < S; jp += kDepCols) {
-    constexpr int N = S < kDepCols ? S : kDepCols;   // words per lane and tile
+  for (int jp = 0; jp < S; jp += N) {
 #pragma unroll
     for (int i = 0; i < N * U; ++i) dep[64 * i + lane] = 0;
     wave_lds_sync();
@@ -300,6 +287,12 @@ __device__ __forceinline__ void major_filter_group(const MV& mv, const MajorTarg
       }
     }
     wave_lds_sync();   // every lane has read its words before they are cleared again
+    if (STEP) {
+      uint32_t live = 0;
+#pragma unroll
+      for (int u = 0; u < U; ++u) live |= cand[u];
+      if (__ballot(live != 0) == 0) return;   // res is 0 still
+    }
   }
   auto any_live = [&]() {
     uint32_t live = 0;

@@ -511,3 +511,59 @@ def test_batch_fold_time(ctx):
         b.free()
     assert us[N.BUFF_Q_SUM, 1 << 24] < 1.5 * us[N.BUFF_Q_GT, 1 << 24], us
     assert us[N.BUFF_Q_MAX, 1 << 22] < 1.2 * us[N.BUFF_Q_SUM, 1 << 22], us
+
+
+# equality on sparse columns: all bytes the majority's with one dense plane or none, a first or a later byte that is not,
+# bytes that no row has together; tiles of no outlier, one, 64, 65 and hundreds
+@pytest.mark.parametrize("decimals", [1, 2, 3, 6])
+@pytest.mark.parametrize("rows", [2000, 60 * TILE + 13])
+def test_sparse_equality(ctx, decimals, rows):
+    rng = np.random.default_rng(decimals)
+    x = np.round(100.0 + 0.1 * rng.integers(-3, 4, rows), decimals)
+    at = [np.array([5, 7])]   # the leading rows decide which columns are sparse
+    for tile, count in zip(range(2, rows // TILE + 1), (0, 1, 64, 65, 700) * 12):
+        at.append(tile * TILE + rng.choice(min(TILE, rows - tile * TILE), min(count, rows - tile * TILE), replace=False))
+    at = np.concatenate(at).astype(int)
+    x[at] = np.round(rng.choice([1e5, 1e5 + 7, 3e5, 7e6], len(at)), decimals)
+    x[5], x[7], x[0] = 7e6, 1e5, 0.0
+    ch = ctx.encode(x, 10 ** decimals, flags=buff_amd.BUFF_MAJORITY)
+    stream = refcpu.major_encode(x, 10 ** decimals)
+    info = ch.info()
+    assert info.sparse_cols > 0
+    f = fixed(x, info.dlen)
+    for pred in (100.0, float(x[3]), 1e5, 1e5 + 7, 3e5, 7e6, 3e5 + 7, 5e6, 0.0):
+        want = f == fixed(pred, info.dlen)
+        words, count = ch.filter("equal", pred, flags=buff_amd.BUFF_SEMANTIC)
+        assert np.array_equal(bits(words, rows), want) and count == want.sum(), (pred, info.sparse_cols)
+        words, count = ch.filter("equal", pred)
+        w_ref, c_ref = refcpu.major_filter(stream, 10 ** decimals, "equal", pred)[:2]
+        assert count == c_ref and np.array_equal(words, w_ref), (pred, info.sparse_cols)
+    ch.free()
+
+
+# an outlier's value where a tile has more than 64 outliers against the majority's value, which reads every dense plane
+def test_sparse_equality_time(ctx):
+    rows = 1 << 26
+    rng = np.random.default_rng(2)
+    base = np.round(100.0 + 0.01 * rng.standard_normal(1 << 20), 3)
+    hit = rng.random(1 << 20) < 0.09
+    base[hit] = np.round(10.0 ** rng.uniform(6, 9, int(hit.sum())), 3)
+    x = np.tile(base, rows >> 20)
+    x[0], x[1] = 0.0, 1e9
+    ch = ctx.encode(x, 1000, flags=buff_amd.BUFF_MAJORITY)
+    assert ch.info().sparse_cols >= 2
+    words = ctx.alloc(rows // 8)
+    us = []
+    for pred in (float(base[hit][3]), float(base[~hit][3])):
+        best = np.inf
+        for _ in range(8):
+            ctx.prof_reset()
+            ctx.prof_enable(True)
+            ch.filter_device("equal", pred, words.ptr, flags=buff_amd.BUFF_SEMANTIC)
+            ctx.synchronize()
+            best = min(best, ctx.prof_query("k_major_filter_eq")[1] * 1e3)
+            ctx.prof_enable(False)
+        us.append(best)
+    for b in (ch, words):
+        b.free()
+    assert us[0] < 1.08 * us[1], us
