@@ -567,3 +567,30 @@ def test_sparse_equality_time(ctx):
     for b in (ch, words):
         b.free()
     assert us[0] < 1.08 * us[1], us
+
+
+# the reference's decode of sparse columns (a later column's majority byte at twice its shift, up to its last outlier):
+# tiles of no outlier, one, 64, 65 and hundreds; the last outlier at either end of a lane's 16 rows and between
+@pytest.mark.parametrize("decimals", [1, 2, 3, 4])
+@pytest.mark.parametrize("last", [0, 1, 7, 15])
+def test_sparse_decode_reference(ctx, decimals, last):
+    rows = 60 * TILE + 13
+    rng = np.random.default_rng(decimals)
+    x = np.round(100.0 + 0.1 * rng.integers(-3, 4, rows), decimals)
+    at = [np.array([5, 7])]   # the leading rows decide which columns are sparse
+    for tile, count in zip(range(2, 50), (0, 1, 64, 65, 700) * 10):
+        at.append(tile * TILE + rng.choice(TILE, count, replace=False))
+    at = np.concatenate(at + [[52 * TILE + 16 * 21 + last]]).astype(int)
+    x[at] = np.round(rng.choice([1e5, 1e5 + 7, 3e5, 7e6], len(at)), decimals)
+    x[at[-1]], x[5], x[7], x[0] = 3e5 + 1, 7e6, 1e5, 0.0
+    ch = ctx.encode(x, 10 ** decimals, flags=buff_amd.BUFF_MAJORITY)
+    assert ch.info().sparse_cols > 0
+    assert {ch.sparse_col(j)[2] for j in range(ch.info().sparse_cols)} & {int(at[-1])}
+    try:
+        want = refcpu.major_decode(refcpu.major_encode(x, 10 ** decimals), 10 ** decimals)
+    except refcpu.RefPanic:
+        with pytest.raises(N.RefPanic):
+            ch.materialize()
+    else:
+        assert np.array_equal(ch.materialize().view(np.uint64), want.view(np.uint64))
+    ch.free()
