@@ -1083,7 +1083,7 @@ def main():
     args = parse()
     if args.gpus != 1:
         print("bench.py measures one GPU: every GPU box here has one MI355X, and this build has no multi-GPU path "
-              "(chunks shard independently; the design is in DESIGN.md). Run with --gpus 1.", file=sys.stderr)
+              "(chunks shard independently). Run with --gpus 1.", file=sys.stderr)
         sys.exit(2)
 
     import buff_amd
